@@ -233,6 +233,39 @@ int dflash_moe_w4a16_noalloc(const void* hidden, int64_t tokens, int64_t hidden_
                              void* stream);
 
 /*
+ * A GDN layer's mixer between its residual adds (model/qwen35_moe_dflash/fused/model.py:206-263), head dims
+ * 128, four conv taps, fp32 inside:
+ *   mid = hidden + out_proj(gated_norm(delta_rule(conv(in_proj(norm(hidden))))));  normed = bf16(post_norm(mid))
+ * in_proj rows are q | k | v | z | b | a (2 * 128 * key_heads + 2 * 128 * value_heads + 2 * value_heads), out_proj is
+ * [hidden_size][128 * value_heads].  Norm weights are applied as w + 1 (input_norm, post_norm) and w (norm).
+ * Outputs besides mid fp32 [T][hidden_size] and normed bf16: what commits any prefix of the block needs --
+ * window bf16 [C][3 + T] (conv history, then the block's columns; C = 128 * (2 * key_heads + value_heads)),
+ * keys, u, core fp32 [value_heads][T][128], cum fp32 [value_heads][T] (log decay summed inside each chunk of 16
+ * tokens) and states fp32 [ceil(T / 16)][value_heads][128][128] (the state after each chunk).
+ */
+typedef struct dflash_gdn {
+  dflash_w4 in_proj, out_proj;
+  const float* input_norm; /* fp32 [hidden_size] */
+  const float* post_norm;  /* fp32 [hidden_size] */
+  const float* norm;       /* fp32 [128] */
+  const float* a_log;      /* fp32 [value_heads] */
+  const float* dt_bias;    /* fp32 [value_heads] */
+  const void* conv;        /* bf16 [C][4] */
+  int64_t hidden_size, key_heads, value_heads;
+  float eps;
+} dflash_gdn;
+size_t dflash_gdn_workspace_bytes(int64_t tokens, int64_t hidden_size, int64_t key_heads, int64_t value_heads);
+int dflash_gdn_mixer(const dflash_gdn* g, const float* hidden, int64_t tokens, const void* history, const float* state,
+                     float* mid, void* normed, void* window, float* states, float* keys, float* u, float* cum,
+                     float* core, void* workspace, size_t workspace_bytes, void* stream);
+/* Commit of a prefix that ends inside a chunk: the state after the chunk's first `accepted` (1..16) tokens, from the
+ * state before the chunk and its rows of the mixer's keys, u (head_stride elements per head, 128 per token) and cum
+ * (cum_stride per head); and columns [first, first + 3) of the window bf16 [channels][pitch] as the conv history. */
+int dflash_gdn_commit(const float* state, const float* keys, const float* u, const float* cum, int64_t head_stride,
+                      int64_t cum_stride, int64_t heads, int64_t accepted, float* state_out, const void* window,
+                      int64_t pitch, int64_t first, int64_t channels, void* history_out, void* stream);
+
+/*
  * Measurement mode (no counterpart in the reference; for benchmarks and
  * profilers that time one kernel of the layer on its own): while a stage is
  * set, dflash_moe_w4a16 and dflash_moe_experts_w4a16 validate their arguments

@@ -49,6 +49,28 @@ class W4Desc(ctypes.Structure):
 
 _W4P = ctypes.POINTER(W4Desc)
 
+
+class GdnDesc(ctypes.Structure):
+    """``struct dflash_gdn``."""
+
+    _fields_ = [
+        ("in_proj", W4Desc),
+        ("out_proj", W4Desc),
+        ("input_norm", ctypes.c_void_p),
+        ("post_norm", ctypes.c_void_p),
+        ("norm", ctypes.c_void_p),
+        ("a_log", ctypes.c_void_p),
+        ("dt_bias", ctypes.c_void_p),
+        ("conv", ctypes.c_void_p),
+        ("hidden_size", ctypes.c_int64),
+        ("key_heads", ctypes.c_int64),
+        ("value_heads", ctypes.c_int64),
+        ("eps", ctypes.c_float),
+    ]
+
+
+_GDNP = ctypes.POINTER(GdnDesc)
+
 SIGNATURES = {
     "dflash_abi_version": (ctypes.c_int, []),
     "dflash_w4_to_tiled": (ctypes.c_int, [_W4P, _P, _P, _P]),
@@ -68,6 +90,9 @@ SIGNATURES = {
                                         _P, _P, _P, _P, _SZ, _P]),
     "dflash_moe_w4a16_noalloc": (ctypes.c_int, [_P, _I64, _I64, _P, _P, _I64, _W4P, _W4P, _W4P, _W4P, _P, _P, _P, _P,
                                                 _P, _P, _P, _P, _P]),
+    "dflash_gdn_workspace_bytes": (_SZ, [_I64, _I64, _I64, _I64]),
+    "dflash_gdn_mixer": (ctypes.c_int, [_GDNP, _P, _I64, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _SZ, _P]),
+    "dflash_gdn_commit": (ctypes.c_int, [_P, _P, _P, _P, _I64, _I64, _I64, _I64, _P, _P, _I64, _I64, _I64, _P, _P]),
     "dflash_set_split_down": (ctypes.c_int, [ctypes.c_int]),
     "dflash_set_tile_pieces": (ctypes.c_int, [ctypes.c_int]),
     "dflash_moe_split_down": (ctypes.c_int, [_I64, _I64, _I64, _I64, _I64, _I64, ctypes.c_int, ctypes.c_int32,

@@ -5,6 +5,7 @@
 // synchronisation, no C++ exception crosses the ABI.
 #include <algorithm>
 #include <atomic>
+#include <initializer_list>
 #include <mutex>
 #include <string>
 
@@ -806,6 +807,129 @@ int dflash_qlinear_w4a16(const void* x, int64_t m, const dflash_w4* weight, void
 int dflash_qlinear_w4a16_f32(const void* x, int64_t m, const dflash_w4* weight, float* y, void* workspace,
                              size_t workspace_bytes, void* stream) {
   return qlinear_impl(x, m, weight, y, true, workspace, workspace_bytes, stream);
+}
+
+namespace {
+struct GdnLayout {
+  size_t normed, proj, gated, mixed, lin, u0, w, qt, kt, pmat, decay, total;
+};
+GdnLayout gdn_layout(int64_t T, int64_t H, int64_t Hk, int64_t Hv) {
+  GdnLayout L;
+  Carver c;
+  const int64_t chunks = (T + 15) / 16, vw = 128 * Hv;
+  const size_t rows = 4 * static_cast<size_t>(Hv) * chunks * 16 * 128;
+  L.normed = c.take(2 * static_cast<size_t>(T) * H);
+  L.proj = c.take(2 * static_cast<size_t>(T) * (256 * Hk + 2 * vw + 2 * Hv));
+  L.gated = c.take(2 * static_cast<size_t>(T) * vw);
+  L.mixed = c.take(2 * static_cast<size_t>(T) * H);
+  L.lin = c.take(std::max(dflash_qlinear_workspace_bytes(T, H, 128), dflash_qlinear_workspace_bytes(T, vw, 128)));
+  L.u0 = c.take(rows);
+  L.w = c.take(rows);
+  L.qt = c.take(rows);
+  L.kt = c.take(rows);
+  L.pmat = c.take(4 * static_cast<size_t>(Hv) * chunks * 256);
+  L.decay = c.take(4 * static_cast<size_t>(Hv) * chunks);
+  L.total = c.off;
+  return L;
+}
+bool mixer_args_aligned(std::initializer_list<const void*> ptrs) {
+  for (const void* q : ptrs)
+    if (!q || !aligned16(q)) return false;
+  return true;
+}
+}  // namespace
+
+size_t dflash_gdn_workspace_bytes(int64_t tokens, int64_t hidden_size, int64_t key_heads, int64_t value_heads) {
+  if (tokens < 0 || hidden_size <= 0 || key_heads <= 0 || value_heads <= 0) return 0;
+  return gdn_layout(tokens, hidden_size, key_heads, value_heads).total;
+}
+
+int dflash_gdn_mixer(const dflash_gdn* g, const float* hidden, int64_t tokens, const void* history, const float* state,
+                     float* mid, void* normed, void* window, float* states, float* keys, float* u, float* cum,
+                     float* core, void* workspace, size_t workspace_bytes, void* stream) {
+  try {
+    if (!g) return fail(DFLASH_ERR_INVALID_ARGUMENT, "gdn: descriptor is NULL");
+    const int64_t T = tokens, H = g->hidden_size, Hk = g->key_heads, Hv = g->value_heads;
+    if (T < 0 || T > (1 << 19)) return fail(DFLASH_ERR_UNSUPPORTED, "gdn: tokens must be in [0, 2^19]");
+    if (Hk <= 0 || Hv <= 0 || Hv % Hk || Hv > 1024)
+      return fail(DFLASH_ERR_UNSUPPORTED, "gdn: value heads must be a multiple of key heads, at most 1024");
+    if (H <= 0 || H % 512 || H > dflash::kMaxNormWidth)
+      return fail(DFLASH_ERR_UNSUPPORTED, "gdn: hidden_size must be a multiple of 512, at most 8192");
+    const int64_t vw = 128 * Hv, n_in = 256 * Hk + 2 * vw + 2 * Hv;
+    if (int r = check_w4(&g->in_proj, "gdn in_proj", 1, n_in, H)) return r;
+    if (int r = check_w4(&g->out_proj, "gdn out_proj", 1, H, vw)) return r;
+    if (T == 0) return DFLASH_OK;
+    if (!mixer_args_aligned({g->input_norm, g->post_norm, g->norm, g->conv, hidden, history, state, mid, normed, window,
+                             states, keys, u, cum, core}) || !g->a_log || !g->dt_bias)
+      return fail(DFLASH_ERR_INVALID_ARGUMENT, "gdn: NULL or misaligned pointer");
+    const GdnLayout L = gdn_layout(T, H, Hk, Hv);
+    if (!workspace || workspace_bytes < L.total || !aligned16(workspace))
+      return fail(DFLASH_ERR_WORKSPACE, "gdn workspace needs " + std::to_string(L.total) + " bytes");
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    uint16_t* x = at<uint16_t>(workspace, L.normed);
+    dflash::GdnParams p{};
+    uint16_t* proj = at<uint16_t>(workspace, L.proj);
+    p.proj = proj;
+    p.ldp = static_cast<int>(n_in);
+    p.T = static_cast<int>(T);
+    p.Hk = static_cast<int>(Hk);
+    p.Hv = static_cast<int>(Hv);
+    p.chunks = static_cast<int>((T + 15) / 16);
+    p.hist = static_cast<const uint16_t*>(history);
+    p.conv = static_cast<const uint16_t*>(g->conv);
+    p.a_log = g->a_log;
+    p.dt_bias = g->dt_bias;
+    p.norm = g->norm;
+    p.eps = g->eps;
+    p.state = state;
+    p.window = static_cast<uint16_t*>(window);
+    p.keys = keys;
+    p.u = u;
+    p.cum = cum;
+    p.core = core;
+    p.states = states;
+    p.u0 = at<float>(workspace, L.u0);
+    p.w = at<float>(workspace, L.w);
+    p.qt = at<float>(workspace, L.qt);
+    p.kt = at<float>(workspace, L.kt);
+    p.pmat = at<float>(workspace, L.pmat);
+    p.decay = at<float>(workspace, L.decay);
+    p.gated = at<uint16_t>(workspace, L.gated);
+    uint16_t* mixed = at<uint16_t>(workspace, L.mixed);
+    void* lin = at<char>(workspace, L.lin);
+    const size_t lin_bytes = L.u0 - L.lin;
+    const int Ti = static_cast<int>(T), Hi = static_cast<int>(H);
+    dflash::launch_add_norm(hidden, nullptr, g->input_norm, g->eps, Ti, Hi, nullptr, x, st);
+    if (int r = launch_status("gdn norm")) return r;
+    if (int r = qlinear_impl(x, T, &g->in_proj, proj, false, lin, lin_bytes, stream)) return r;
+    dflash::launch_gdn(p, st);
+    if (int r = launch_status("gdn")) return r;
+    if (int r = qlinear_impl(p.gated, T, &g->out_proj, mixed, false, lin, lin_bytes, stream)) return r;
+    dflash::launch_add_norm(hidden, mixed, g->post_norm, g->eps, Ti, Hi, mid, static_cast<uint16_t*>(normed), st);
+    return launch_status("gdn norm");
+  } catch (...) {
+    return fail(DFLASH_ERR_HIP, "unexpected host exception");
+  }
+}
+
+int dflash_gdn_commit(const float* state, const float* keys, const float* u, const float* cum, int64_t head_stride,
+                      int64_t cum_stride, int64_t heads, int64_t accepted, float* state_out, const void* window,
+                      int64_t pitch, int64_t first, int64_t channels, void* history_out, void* stream) {
+  try {
+    if (heads <= 0 || heads > 1024 || accepted < 1 || accepted > 16 || head_stride < accepted * 128 ||
+        cum_stride < accepted || channels <= 0 || channels > (1 << 24) || first < 0 || first + 3 > pitch ||
+        first > (1 << 24))
+      return fail(DFLASH_ERR_INVALID_ARGUMENT, "gdn_commit: heads, accepted, strides or window out of range");
+    if (!state || !keys || !u || !cum || !state_out || !window || !history_out)
+      return fail(DFLASH_ERR_INVALID_ARGUMENT, "gdn_commit: NULL pointer");
+    dflash::launch_gdn_commit(state, keys, u, cum, head_stride, cum_stride, static_cast<int>(heads),
+                              static_cast<int>(accepted), state_out, static_cast<const uint16_t*>(window), pitch,
+                              static_cast<int>(first), static_cast<int>(channels), static_cast<uint16_t*>(history_out),
+                              static_cast<hipStream_t>(stream));
+    return launch_status("gdn_commit");
+  } catch (...) {
+    return fail(DFLASH_ERR_HIP, "unexpected host exception");
+  }
 }
 
 int dflash_router_logits(const void* hidden, int64_t tokens, int64_t hidden_size, const void* router_weight,

@@ -276,4 +276,39 @@ void launch_w4_small(const SmallLinearParams& p, hipStream_t stream);
 bool small_linear_stream_fits(int M, int N, int K, int G);
 void launch_w4_small_stream(const SmallLinearParams& p, int grid, hipStream_t stream);
 
+// Gated-DeltaNet mixer around its projections (gdn.hip): head dims 128, four conv taps.
+constexpr int kMaxNormWidth = 8192;  // row width launch_add_norm takes (a multiple of 4)
+// mid = hidden + mixed (mixed null: mid not written), normed = bf16(rms(mid) * (w + 1)); rows of H columns
+void launch_add_norm(const float* hidden, const uint16_t* mixed, const float* w, float eps, int T, int H, float* mid,
+                     uint16_t* normed, hipStream_t stream);
+struct GdnParams {
+  const uint16_t* proj;    // bf16 [T][ldp]: q | k | v | z | b | a
+  int ldp;
+  int T, Hk, Hv, chunks;   // chunks of 16 tokens
+  const uint16_t* hist;    // bf16 [C][3] conv history
+  const uint16_t* conv;    // bf16 [C][4] taps
+  const float* a_log;      // [Hv]
+  const float* dt_bias;    // [Hv]
+  const float* norm;       // [128] gated norm weight
+  float eps;
+  const float* state;      // [Hv][128][128] before the block
+  // kept by the caller
+  uint16_t* window;        // bf16 [C][3 + T]
+  float* keys;             // [Hv][T][128] normalised keys
+  float* u;                // [Hv][T][128] delta-rule writes
+  float* cum;              // [Hv][T] log decay summed inside each chunk
+  float* core;             // [Hv][T][128]
+  float* states;           // [chunks][Hv][128][128] after each chunk
+  // scratch, per (head, chunk): 16 x 128 each (u0 and kt column by column), the 16 x 16 output mixing matrix and
+  // the chunk's decay
+  float *u0, *w, *qt, *kt, *pmat, *decay;
+  uint16_t* gated;         // bf16 [T][Hv * 128]
+};
+void launch_gdn(const GdnParams& p, hipStream_t stream);
+// State after the first j >= 1 tokens of one chunk (state before it, its keys, u and cum; strides in elements per head), and
+// columns [first, first + 3) of the window [channels][pitch] as the conv history
+void launch_gdn_commit(const float* state, const float* keys, const float* u, const float* cum, int64_t row_stride,
+                       int64_t cum_stride, int heads, int j, float* out, const uint16_t* window, int64_t pitch, int first,
+                       int channels, uint16_t* hist, hipStream_t stream);
+
 }  // namespace dflash

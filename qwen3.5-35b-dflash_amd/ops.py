@@ -143,6 +143,98 @@ def qlinear(x: torch.Tensor, weight: PackedW4, *, workspace: Optional[torch.Tens
     return out.reshape(*x.shape[:-1], weight.rows)
 
 
+class GdnMixer(NamedTuple):
+    """Outputs of :func:`gdn_mixer` (see ``dflash_gdn_mixer`` in ``include/dflash_hip.h``)."""
+
+    mid: torch.Tensor        # fp32 [T, H] residual after the mixer
+    normed: torch.Tensor     # bf16 [T, H] its post-norm
+    window: torch.Tensor     # bf16 [1, C, 3 + T]
+    states: torch.Tensor     # fp32 [chunks, 1, Hv, 128, 128]
+    keys: torch.Tensor       # fp32 [1, Hv, T, 128]
+    u: torch.Tensor          # fp32 [1, Hv, T, 128]
+    cum: torch.Tensor        # fp32 [1, Hv, T]
+    core: torch.Tensor       # fp32 [1, Hv, T, 128]
+
+
+def gdn_mixer(hidden: torch.Tensor, history: torch.Tensor, state: torch.Tensor, *, in_proj: PackedW4,
+              out_proj: PackedW4, input_norm: torch.Tensor, post_norm: torch.Tensor, norm: torch.Tensor,
+              a_log: torch.Tensor, dt_bias: torch.Tensor, conv: torch.Tensor, key_heads: int, eps: float) -> GdnMixer:
+    """A GDN layer from its residual to the MoE input, in one call: norm, in_proj, conv, gated delta rule, gated
+    norm, out_proj, residual add, post-norm.  Tensors as :func:`gdn_mixer_fits` accepts them."""
+    device, t, h = hidden.device, hidden.shape[0], hidden.shape[1]
+    hv = a_log.shape[0]
+    f32 = dict(dtype=torch.float32, device=device)
+    b16 = dict(dtype=torch.bfloat16, device=device)
+    rows = (1, hv, t, 128)
+    r = GdnMixer(torch.empty((t, h), **f32), torch.empty((t, h), **b16),
+                 torch.empty((1, conv.shape[0], 3 + t), **b16),
+                 torch.empty(((t + 15) // 16, 1, hv, 128, 128), **f32), torch.empty(rows, **f32),
+                 torch.empty(rows, **f32), torch.empty((1, hv, t), **f32), torch.empty(rows, **f32))
+    desc = _lib.GdnDesc(_desc(in_proj), _desc(out_proj), input_norm.data_ptr(), post_norm.data_ptr(), norm.data_ptr(),
+                        a_log.data_ptr(), dt_bias.data_ptr(), conv.data_ptr(), h, key_heads, hv, eps)
+    ws = _workspace(_lib.load().dflash_gdn_workspace_bytes(t, h, key_heads, hv), device, None)
+    _lib.call("dflash_gdn_mixer", ctypes.byref(desc), _ptr(hidden), t, _ptr(history), _ptr(state), _ptr(r.mid),
+              _ptr(r.normed), _ptr(r.window), _ptr(r.states), _ptr(r.keys), _ptr(r.u), _ptr(r.cum), _ptr(r.core),
+              _ptr(ws), ws.numel(), _stream(device))
+    return r
+
+
+def _as(t, dtype: torch.dtype, shape: tuple, device: torch.device) -> bool:
+    """Whether ``t`` is what a kernel reads as is: this dtype, shape and device, contiguous, 16-byte aligned."""
+    return (isinstance(t, torch.Tensor) and t.dtype == dtype and t.shape == shape and t.device == device
+            and t.is_contiguous() and t.data_ptr() % 16 == 0)
+
+
+def _matrix(w, rows: int, cols: int, device: torch.device) -> bool:
+    """Whether ``w`` is a valid packed matrix of this size on this device."""
+    if not isinstance(w, PackedW4) or w.packed.ndim != 2 or (w.rows, w.cols) != (rows, cols):
+        return False
+    w.validate("weight")
+    return w.packed.device == device
+
+
+def gdn_mixer_fits(hidden: torch.Tensor, history: torch.Tensor, state: torch.Tensor, *, in_proj: PackedW4,
+                   out_proj: PackedW4, input_norm: torch.Tensor, post_norm: torch.Tensor, norm: torch.Tensor,
+                   a_log: torch.Tensor, dt_bias: torch.Tensor, conv: torch.Tensor, key_heads: int, eps: float) -> bool:
+    """Whether :func:`gdn_mixer` takes these arguments: head dims 128, four taps, plain contiguous tensors of the
+    dtypes the target keeps, at least one token, and no gradient asked for."""
+    device = hidden.device
+    if (device.type != "cuda" or hidden.ndim != 2 or hidden.dtype != torch.float32 or not hidden.is_contiguous()
+            or hidden.shape[0] < 1 or hidden.shape[0] > 1 << 19 or hidden.data_ptr() % 16
+            or (hidden.requires_grad and torch.is_grad_enabled())):
+        return False
+    h, hv, f32, b16 = hidden.shape[1], a_log.shape[0], torch.float32, torch.bfloat16
+    width = 128 * (2 * key_heads + hv)
+    return (h % 512 == 0 and h <= 8192 and hv <= 1024 and hv % key_heads == 0
+            and _as(history, b16, (1, width, 3), device) and _as(state, f32, (1, hv, 128, 128), device)
+            and _as(conv, b16, (width, 1, 4), device) and _as(norm, f32, (128,), device)
+            and _as(input_norm, f32, (h,), device) and _as(post_norm, f32, (h,), device)
+            and _as(a_log, f32, (hv,), device) and _as(dt_bias, f32, (hv,), device)
+            and _matrix(in_proj, width + 128 * hv + 2 * hv, h, device) and _matrix(out_proj, h, 128 * hv, device))
+
+
+def gdn_commit(state: torch.Tensor, keys: torch.Tensor, u: torch.Tensor, cum: torch.Tensor, accepted: int,
+               window: torch.Tensor, first: int) -> Optional[tuple]:
+    """``(recurrent state, conv history)`` after the first ``accepted`` tokens of one chunk of :func:`gdn_mixer`
+    (``layers.state_after`` and the window's columns ``[first, first + 3)``) in one launch; ``None`` when the tensors
+    are not laid out as that call leaves them."""
+    hv, device = state.shape[1], state.device
+    if (device.type != "cuda" or not 1 <= accepted <= 16 or not _as(state, torch.float32, (1, hv, 128, 128), device)
+            or keys.shape[:2] != (1, hv) or keys.shape[2] < accepted or keys.shape[3] != 128 or u.shape != keys.shape
+            or cum.shape != keys.shape[:3]
+            or any(t.dtype != torch.float32 or t.device != device for t in (keys, u, cum))
+            or keys.stride()[2:] != (128, 1) or u.stride() != keys.stride() or cum.stride(2) != 1
+            or window.dtype != torch.bfloat16 or window.ndim != 3 or window.shape[0] != 1 or window.device != device
+            or not window.is_contiguous() or first + 3 > window.shape[2]):
+        return None
+    out = torch.empty_like(state)
+    history = torch.empty((1, window.shape[1], 3), dtype=window.dtype, device=device)
+    _lib.call("dflash_gdn_commit", _ptr(state), _ptr(keys), _ptr(u), _ptr(cum), keys.stride(1), cum.stride(1), hv,
+              accepted, _ptr(out), _ptr(window), window.shape[2], first, window.shape[1], _ptr(history),
+              _stream(device))
+    return out, history
+
+
 def router_logits(hidden: torch.Tensor, router_weight: torch.Tensor) -> torch.Tensor:
     """fp32 ``[T, E]`` logits from bf16 ``hidden [..., H]`` and bf16 ``router_weight [E, H]``."""
     device = _require_device(hidden, router_weight)

@@ -303,11 +303,38 @@ class TargetModel:
         return ops.moe_w4a16(x, lw.gate_up, lw.down, top_k=self.config.top_k, router_weight=lw.router,
                              shared=lw.shared, workspace=workspace)
 
+    def _gdn_args(self, lw: LayerWeights) -> dict:
+        c = self.config
+        return dict(in_proj=lw.mixer_in, out_proj=lw.mixer_out, input_norm=lw.input_norm, post_norm=lw.post_norm,
+                    norm=lw.gdn_norm, a_log=lw.a_log, dt_bias=lw.dt_bias, conv=lw.conv, key_heads=c.linear_key_heads,
+                    eps=c.rms_eps)
+
+    def _gdn_kernels(self, hidden: Tensor, lw: LayerWeights, conv_hist: Tensor, state: Tensor):
+        """The mixer half of a GDN layer on the HIP kernels: ``(mid, moe input, pending)``, or ``None`` when
+        the layer is not one they take (``ops.gdn_mixer_fits``)."""
+        c, args = self.config, self._gdn_args(lw)
+        if c.linear_key_dim != 128 or c.linear_value_dim != 128 or c.linear_value_heads != lw.a_log.shape[0]:
+            return None
+        if not ops.gdn_mixer_fits(hidden, conv_hist, state, **args):
+            return None
+        r = ops.gdn_mixer(hidden, conv_hist, state, **args)
+        n = layers.CHUNK
+        chunks = [layers.DeltaChunk(*f) for f in zip(r.core.split(n, 2), r.states.unbind(0), r.keys.split(n, 2),
+                                                     r.u.split(n, 2), r.cum.split(n, 2))]
+        return r.mid, r.normed, GdnPending(r.window, state, chunks)
+
     def layer(self, i: int, hidden: Tensor, state: TargetState, workspace: Optional[Tensor] = None,
               trace: Optional[dict] = None):
         """One decoder layer on the fp32 residual ``[T, H]``; returns (hidden, GdnPending or None).
         ``trace`` (a dict) receives the residual after the mixer and the MoE input."""
         c, lw = self.config, self.w.layers[i]
+        if lw.kind == "linear_attention":
+            done = self._gdn_kernels(hidden, lw, state.conv[i], state.recurrent[i])
+            if done is not None:
+                mid, normed, pending = done
+                if trace is not None:
+                    trace.update(mid=mid, moe_in=normed)
+                return mid + self._moe(normed, lw, workspace), pending     # bf16 joins the fp32 sum exactly
         normed = layers.rms_normalise(hidden, lw.input_norm, c.rms_eps, 1.0).to(torch.bfloat16)
         pending = None
         if lw.kind == "linear_attention":
@@ -356,13 +383,19 @@ class TargetModel:
         for i, p in enumerate(pending.gdn):
             if p is None:
                 continue
-            state.conv[i] = p.window[:, :, accepted:accepted + keep].clone()
             full, rest = divmod(accepted, layers.CHUNK)
-            s = p.state
-            for ch in p.chunks[:full]:
-                s = ch.state
+            if accepted == pending.tokens:                  # the whole block: a short last chunk ends there too
+                full, rest = len(p.chunks), 0
+            s = p.chunks[full - 1].state if full else p.state
             if rest:
                 ch = p.chunks[full]
+                done = ops.gdn_commit(s, ch.keys, ch.u, ch.cum, rest, p.window, accepted) if keep == 3 else None
+                if done is not None:
+                    state.recurrent[i], state.conv[i] = done
+                    continue
                 s = layers.state_after(s, ch.keys, ch.u, ch.cum, rest)
-            state.recurrent[i] = s.clone() if s is p.state else s
+            state.conv[i] = p.window[:, :, accepted:accepted + keep].clone()
+            # a state of its own: not the one before the block, nor a view that keeps every chunk's alive
+            whole = s.untyped_storage().nbytes() == s.nbytes
+            state.recurrent[i] = s if s is not p.state and whole else s.clone()
         state.position += accepted

@@ -1,0 +1,61 @@
+"""GPU: the mixer kernels of a decoder layer against the decoder-layer oracle (``oracle/stack.py``).
+
+The lengths are those where the GDN kernels can go wrong: one token, a chunk one short, full and one over, a ragged
+last chunk; value heads per key head 1 and 4.  The oracle follows the rule token by token in float64 on the
+bf16-rounded projections, so what differs is the order of fp32 sums and the bf16 rounding of
+the two projections: outputs within one bf16 ulp of a projection that rounds the other way.  bf16 keeps 8 significant
+bits, so an ulp of a value in [2^e, 2^(e+1)) is 2^(e-7), at most 2^-7 of the largest value.
+"""
+import pytest
+import torch
+
+from oracle import metrics, stack
+from stack_util import oracle_layer_state, oracle_layer_weights
+
+pytestmark = pytest.mark.gpu
+TOL = 2.0 ** -7
+
+
+def _gdn_model(pkg, device, key_heads, value_heads, tokens):
+    base = pkg.target.small_config(("linear_attention",))
+    c = type(base)(**{**vars(base), "linear_key_heads": key_heads, "linear_value_heads": value_heads})
+    host = pkg.target.random_weights(c, seed=7, device="cpu", layout="portable", generate_on="cpu")
+    layout = "tiled" if tokens <= 32 else "portable"
+    model = pkg.target.TargetModel(pkg.target.to_device(host, device, layout=layout), capacity=96)
+    return c, host, model, model.synthetic_context(5, seed=8)
+
+
+@pytest.mark.parametrize("key_heads,value_heads", [(4, 16), (16, 16)])
+@pytest.mark.parametrize("tokens", [1, 3, 15, 16, 17, 32, 41])
+def test_gdn_layer_matches_oracle(pkg, device, tokens, key_heads, value_heads):
+    c, host, model, state = _gdn_model(pkg, device, key_heads, value_heads, tokens)
+    x = torch.randn((tokens, c.hidden), generator=torch.Generator().manual_seed(tokens))
+    assert pkg.ops.gdn_mixer_fits(x.to(device), state.conv[0], state.recurrent[0], **model._gdn_args(model.w.layers[0]))
+    trace = {}
+    _, pending = model.layer(0, x.to(device), state, trace=trace)
+    lw = oracle_layer_weights(host.layers[0])
+    before = oracle_layer_state(state, 0)
+    normed = stack.bf16(stack.norm(x, lw["input_norm"], c.rms_eps, 1.0))
+    ref = stack.gdn_layer(normed, lw, before["conv"], before["recurrent"], c)
+    mid = x + ref["out"]
+    print(f"gdn T={tokens} {key_heads}/{value_heads}", metrics.compare(trace["mid"].cpu(), mid), flush=True)
+    assert metrics.compare(trace["mid"].cpu(), mid)["max_rel"] <= TOL
+    want = stack.bf16(stack.norm(trace["mid"].cpu(), lw["post_norm"], c.rms_eps, 1.0))
+    assert metrics.compare(trace["moe_in"].float().cpu(), want)["max_rel"] <= TOL
+    assert metrics.compare(pending.window[0].float().cpu(), ref["window"])["max_rel"] <= TOL
+    for j in sorted({1, tokens // 2, tokens - 1, tokens} - {0}):
+        trial = state.clone()
+        model.commit(trial, pkg.target.Pending(state.position, tokens, [pending]), j)
+        assert metrics.compare(trial.recurrent[0][0].cpu(), ref["states"][j].float())["max_rel"] <= TOL, j
+        assert torch.equal(trial.conv[0], pending.window[:, :, j:j + 3])
+
+
+def test_gdn_layer_takes_the_general_path_for_other_forms(pkg, device):
+    """A conv history that is a strided view gives the result of its contiguous copy."""
+    c, _, model, state = _gdn_model(pkg, device, 4, 16, 16)
+    x = torch.randn((16, c.hidden), generator=torch.Generator().manual_seed(3)).to(device)
+    want, _ = model.layer(0, x, state)
+    state.conv[0] = state.conv[0].transpose(1, 2).contiguous().transpose(1, 2)
+    assert not pkg.ops.gdn_mixer_fits(x, state.conv[0], state.recurrent[0], **model._gdn_args(model.w.layers[0]))
+    got, _ = model.layer(0, x, state)
+    assert metrics.compare(got.cpu(), want.cpu())["max_rel"] <= TOL
