@@ -266,6 +266,31 @@ int dflash_gdn_commit(const float* state, const float* keys, const float* u, con
                       int64_t pitch, int64_t first, int64_t channels, void* history_out, void* stream);
 
 /*
+ * A full-attention layer's mixer between its residual adds (model/qwen35_moe_dflash/fused/model.py:265-294), head
+ * dims 128 and 256, fp32 inside over a bf16 cache:
+ *   mid = hidden + out_proj(sigmoid(gate) * attention(rotary(norm(q)), cache)), q | gate | k | v = in_proj(norm(hidden));
+ *   normed = bf16(post_norm(mid)).
+ * in_proj rows are per head query | gate (2 * head_dim), then the K heads, then the V heads; out_proj is
+ * [hidden_size][heads * head_dim].  Norm weights are applied as w + 1.  The block's K and V rows are written to rows
+ * [position, position + T) of the caches bf16 [kv_heads][capacity][head_dim]; token t sees rows <= position + t.
+ */
+typedef struct dflash_attention {
+  dflash_w4 in_proj, out_proj;
+  const float* input_norm; /* fp32 [hidden_size] */
+  const float* post_norm;  /* fp32 [hidden_size] */
+  const float* q_norm;     /* fp32 [head_dim] */
+  const float* k_norm;     /* fp32 [head_dim] */
+  const float* inv_freq;   /* fp32 [rotary_dim / 2] */
+  int64_t hidden_size, heads, kv_heads, head_dim, rotary_dim;
+  float eps;
+} dflash_attention;
+size_t dflash_attention_workspace_bytes(int64_t tokens, int64_t hidden_size, int64_t heads, int64_t kv_heads,
+                                        int64_t head_dim);
+int dflash_attention_mixer(const dflash_attention* a, const float* hidden, int64_t tokens, int64_t position,
+                           void* keys, void* values, int64_t capacity, float* mid, void* normed, void* workspace,
+                           size_t workspace_bytes, void* stream);
+
+/*
  * Measurement mode (no counterpart in the reference; for benchmarks and
  * profilers that time one kernel of the layer on its own): while a stage is
  * set, dflash_moe_w4a16 and dflash_moe_experts_w4a16 validate their arguments

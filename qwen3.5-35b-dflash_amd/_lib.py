@@ -69,7 +69,28 @@ class GdnDesc(ctypes.Structure):
     ]
 
 
+class AttentionDesc(ctypes.Structure):
+    """``struct dflash_attention``."""
+
+    _fields_ = [
+        ("in_proj", W4Desc),
+        ("out_proj", W4Desc),
+        ("input_norm", ctypes.c_void_p),
+        ("post_norm", ctypes.c_void_p),
+        ("q_norm", ctypes.c_void_p),
+        ("k_norm", ctypes.c_void_p),
+        ("inv_freq", ctypes.c_void_p),
+        ("hidden_size", ctypes.c_int64),
+        ("heads", ctypes.c_int64),
+        ("kv_heads", ctypes.c_int64),
+        ("head_dim", ctypes.c_int64),
+        ("rotary_dim", ctypes.c_int64),
+        ("eps", ctypes.c_float),
+    ]
+
+
 _GDNP = ctypes.POINTER(GdnDesc)
+_ATTNP = ctypes.POINTER(AttentionDesc)
 
 SIGNATURES = {
     "dflash_abi_version": (ctypes.c_int, []),
@@ -93,6 +114,8 @@ SIGNATURES = {
     "dflash_gdn_workspace_bytes": (_SZ, [_I64, _I64, _I64, _I64]),
     "dflash_gdn_mixer": (ctypes.c_int, [_GDNP, _P, _I64, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _SZ, _P]),
     "dflash_gdn_commit": (ctypes.c_int, [_P, _P, _P, _P, _I64, _I64, _I64, _I64, _P, _P, _I64, _I64, _I64, _P, _P]),
+    "dflash_attention_workspace_bytes": (_SZ, [_I64, _I64, _I64, _I64, _I64]),
+    "dflash_attention_mixer": (ctypes.c_int, [_ATTNP, _P, _I64, _I64, _P, _P, _I64, _P, _P, _P, _SZ, _P]),
     "dflash_set_split_down": (ctypes.c_int, [ctypes.c_int]),
     "dflash_set_tile_pieces": (ctypes.c_int, [ctypes.c_int]),
     "dflash_moe_split_down": (ctypes.c_int, [_I64, _I64, _I64, _I64, _I64, _I64, ctypes.c_int, ctypes.c_int32,

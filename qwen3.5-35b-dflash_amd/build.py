@@ -21,7 +21,7 @@ LIBRARY = PACKAGE_DIR / "libdflash_hip.so"
 TIMELINE_LIBRARY = PACKAGE_DIR / "libdflash_hip_timeline.so"
 SOURCES = ("csrc/api.hip", "csrc/route.hip", "csrc/w4_gemm.hip", "csrc/w4_stream.hip",
            "csrc/w4_tile.hip", "csrc/w4_verify.hip", "csrc/w4_small.hip",
-           "csrc/repack.hip", "csrc/gdn.hip")
+           "csrc/repack.hip", "csrc/gdn.hip", "csrc/attention.hip")
 ARCH = "gfx950"
 FLAGS = (
     f"--offload-arch={ARCH}", "-O3", "-std=c++17", "-fPIC",

@@ -932,6 +932,106 @@ int dflash_gdn_commit(const float* state, const float* keys, const float* u, con
   }
 }
 
+namespace {
+struct AttnLayout {
+  size_t normed, proj, att, mixed, lin, q, part, ml, total;
+};
+AttnLayout attn_layout(int64_t T, int64_t H, int64_t heads, int64_t kv, int64_t D) {
+  AttnLayout L;
+  Carver c;
+  const int64_t rows = T * (heads / kv);
+  const size_t partial = static_cast<size_t>(dflash::attn_partial_rows(static_cast<int>(rows), static_cast<int>(kv), cu_count()));
+  L.normed = c.take(2 * static_cast<size_t>(T) * H);
+  L.proj = c.take(2 * static_cast<size_t>(T) * (2 * heads * D + 2 * kv * D));
+  L.att = c.take(2 * static_cast<size_t>(T) * heads * D);
+  L.mixed = c.take(2 * static_cast<size_t>(T) * H);
+  L.lin = c.take(std::max(dflash_qlinear_workspace_bytes(T, H, 128), dflash_qlinear_workspace_bytes(T, heads * D, 128)));
+  L.q = c.take(3 * 2 * static_cast<size_t>(T) * heads * D);
+  L.part = c.take(4 * partial * D);
+  L.ml = c.take(8 * partial);
+  L.total = c.off;
+  return L;
+}
+// The shapes the attention kernels take; row counts and cache offsets stay far inside 32 and 64 bits.
+bool attn_shape_ok(int64_t T, int64_t H, int64_t heads, int64_t kv, int64_t D) {
+  return T >= 0 && H > 0 && heads > 0 && kv > 0 && heads % kv == 0 && heads <= 1024 && (D == 128 || D == 256) &&
+         T * heads <= (int64_t(1) << 22);
+}
+}  // namespace
+
+size_t dflash_attention_workspace_bytes(int64_t tokens, int64_t hidden_size, int64_t heads, int64_t kv_heads,
+                                        int64_t head_dim) {
+  if (!attn_shape_ok(tokens, hidden_size, heads, kv_heads, head_dim)) return 0;
+  return attn_layout(tokens, hidden_size, heads, kv_heads, head_dim).total;
+}
+
+int dflash_attention_mixer(const dflash_attention* a, const float* hidden, int64_t tokens, int64_t position,
+                           void* keys, void* values, int64_t capacity, float* mid, void* normed, void* workspace,
+                           size_t workspace_bytes, void* stream) {
+  try {
+    if (!a) return fail(DFLASH_ERR_INVALID_ARGUMENT, "attention: descriptor is NULL");
+    const int64_t T = tokens, H = a->hidden_size, heads = a->heads, kv = a->kv_heads, D = a->head_dim;
+    if (!attn_shape_ok(T, H, heads, kv, D))
+      return fail(DFLASH_ERR_UNSUPPORTED, "attention: head_dim must be 128 or 256, heads a multiple of kv_heads, tokens * heads at most 2^22");
+    if (H % 512 || H > dflash::kMaxNormWidth)
+      return fail(DFLASH_ERR_UNSUPPORTED, "attention: hidden_size must be a multiple of 512, at most 8192");
+    if (a->rotary_dim <= 0 || a->rotary_dim > D || a->rotary_dim % (2 * (D / 64)))
+      return fail(DFLASH_ERR_UNSUPPORTED, "attention: rotary_dim must be a multiple of head_dim / 32, at most head_dim");
+    if (position < 0 || capacity > (1 << 24) || position + T > capacity)
+      return fail(DFLASH_ERR_INVALID_ARGUMENT, "attention: block would exceed the KV cache capacity");
+    const int64_t n_in = 2 * heads * D + 2 * kv * D;
+    if (int r = check_w4(&a->in_proj, "attention in_proj", 1, n_in, H)) return r;
+    if (int r = check_w4(&a->out_proj, "attention out_proj", 1, H, heads * D)) return r;
+    if (T == 0) return DFLASH_OK;
+    if (!mixer_args_aligned({a->input_norm, a->post_norm, a->q_norm, a->k_norm, hidden, keys, values, mid, normed}) ||
+        !a->inv_freq)
+      return fail(DFLASH_ERR_INVALID_ARGUMENT, "attention: NULL or misaligned pointer");
+    const AttnLayout L = attn_layout(T, H, heads, kv, D);
+    if (!workspace || workspace_bytes < L.total || !aligned16(workspace))
+      return fail(DFLASH_ERR_WORKSPACE, "attention workspace needs " + std::to_string(L.total) + " bytes");
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    uint16_t* x = at<uint16_t>(workspace, L.normed);
+    uint16_t* proj = at<uint16_t>(workspace, L.proj);
+    uint16_t* mixed = at<uint16_t>(workspace, L.mixed);
+    dflash::AttnParams p{};
+    p.proj = proj;
+    p.ldp = static_cast<int>(n_in);
+    p.T = static_cast<int>(T);
+    p.heads = static_cast<int>(heads);
+    p.kv = static_cast<int>(kv);
+    p.position = static_cast<int>(position);
+    p.capacity = static_cast<int>(capacity);
+    p.rotary_half = static_cast<int>(a->rotary_dim / 2);
+    p.inv_freq = a->inv_freq;
+    p.q_norm = a->q_norm;
+    p.k_norm = a->k_norm;
+    p.eps = a->eps;
+    p.scale = D == 256 ? 0.0625f : 0.08838834764831845f;  // head_dim^-1/2
+    p.keys = static_cast<uint16_t*>(keys);
+    p.values = static_cast<uint16_t*>(values);
+    const int n = static_cast<int>(position + T), rows = static_cast<int>(T * (heads / kv));
+    p.splits = dflash::attn_splits(rows, p.kv, n, cu_count());
+    p.split_keys = ((n + p.splits - 1) / p.splits + 31) / 32 * 32;
+    p.q = at<uint16_t>(workspace, L.q);
+    p.part = at<float>(workspace, L.part);
+    p.ml = at<float2>(workspace, L.ml);
+    p.out = at<uint16_t>(workspace, L.att);
+    void* lin = at<char>(workspace, L.lin);
+    const size_t lin_bytes = L.q - L.lin;
+    const int Ti = p.T, Hi = static_cast<int>(H);
+    dflash::launch_add_norm(hidden, nullptr, a->input_norm, a->eps, Ti, Hi, nullptr, x, st);
+    if (int r = launch_status("attention norm")) return r;
+    if (int r = qlinear_impl(x, T, &a->in_proj, proj, false, lin, lin_bytes, stream)) return r;
+    dflash::launch_attention(static_cast<int>(D), p, st);
+    if (int r = launch_status("attention")) return r;
+    if (int r = qlinear_impl(p.out, T, &a->out_proj, mixed, false, lin, lin_bytes, stream)) return r;
+    dflash::launch_add_norm(hidden, mixed, a->post_norm, a->eps, Ti, Hi, mid, static_cast<uint16_t*>(normed), st);
+    return launch_status("attention norm");
+  } catch (...) {
+    return fail(DFLASH_ERR_HIP, "unexpected host exception");
+  }
+}
+
 int dflash_router_logits(const void* hidden, int64_t tokens, int64_t hidden_size, const void* router_weight,
                          int64_t experts, float* logits, void* stream) {
   try {

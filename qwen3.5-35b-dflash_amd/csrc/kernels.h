@@ -311,4 +311,25 @@ void launch_gdn_commit(const float* state, const float* keys, const float* u, co
                        int64_t cum_stride, int heads, int j, float* out, const uint16_t* window, int64_t pitch, int first,
                        int channels, uint16_t* hist, hipStream_t stream);
 
+// Attention mixer around its projections (attention.hip): head dims 128 and 256.
+struct AttnParams {
+  const uint16_t* proj;   // bf16 [T][ldp]: per head query | gate, then K heads, V heads
+  int ldp;
+  int T, heads, kv, position, capacity;
+  int rotary_half;        // features that rotate / 2, a multiple of head_dim / 64
+  const float* inv_freq;  // [rotary_half]
+  const float *q_norm, *k_norm;  // [head_dim], applied as w + 1
+  float eps, scale;
+  uint16_t *keys, *values;       // bf16 [kv][capacity][head_dim], rows [position, position + T) written here
+  int splits, split_keys;        // splits * split_keys >= position + T; split_keys a multiple of 32
+  // scratch
+  uint16_t* q;            // bf16 [3][kv][T * group][head_dim]: scaled queries as three parts
+  float* part;            // [splits][kv][T * group][head_dim]
+  float2* ml;             // [splits][kv][T * group]: maximum score, sum of exp(score - maximum)
+  uint16_t* out;          // bf16 [T][heads * head_dim]
+};
+int attn_splits(int rows, int kv, int keys, int cus);
+int64_t attn_partial_rows(int rows, int kv, int cus);  // bound on splits * kv * rows over any number of keys
+void launch_attention(int head_dim, const AttnParams& p, hipStream_t stream);
+
 }  // namespace dflash

@@ -193,19 +193,25 @@ def _matrix(w, rows: int, cols: int, device: torch.device) -> bool:
     return w.packed.device == device
 
 
+def _residual(hidden: torch.Tensor) -> bool:
+    """Whether the mixer kernels take this residual: fp32 ``[T, H]`` as it lies, at least one token, H they can
+    normalise, and no gradient asked for."""
+    return (_as(hidden, torch.float32, hidden.shape, hidden.device) and hidden.is_cuda and hidden.ndim == 2
+            and 1 <= hidden.shape[0] <= 1 << 19 and hidden.shape[1] % 512 == 0 and 512 <= hidden.shape[1] <= 8192
+            and not (hidden.requires_grad and torch.is_grad_enabled()))
+
+
 def gdn_mixer_fits(hidden: torch.Tensor, history: torch.Tensor, state: torch.Tensor, *, in_proj: PackedW4,
                    out_proj: PackedW4, input_norm: torch.Tensor, post_norm: torch.Tensor, norm: torch.Tensor,
                    a_log: torch.Tensor, dt_bias: torch.Tensor, conv: torch.Tensor, key_heads: int, eps: float) -> bool:
     """Whether :func:`gdn_mixer` takes these arguments: head dims 128, four taps, plain contiguous tensors of the
     dtypes the target keeps, at least one token, and no gradient asked for."""
-    device = hidden.device
-    if (device.type != "cuda" or hidden.ndim != 2 or hidden.dtype != torch.float32 or not hidden.is_contiguous()
-            or hidden.shape[0] < 1 or hidden.shape[0] > 1 << 19 or hidden.data_ptr() % 16
-            or (hidden.requires_grad and torch.is_grad_enabled())):
+    if not _residual(hidden):
         return False
+    device = hidden.device
     h, hv, f32, b16 = hidden.shape[1], a_log.shape[0], torch.float32, torch.bfloat16
     width = 128 * (2 * key_heads + hv)
-    return (h % 512 == 0 and h <= 8192 and hv <= 1024 and hv % key_heads == 0
+    return (hv <= 1024 and hv % key_heads == 0
             and _as(history, b16, (1, width, 3), device) and _as(state, f32, (1, hv, 128, 128), device)
             and _as(conv, b16, (width, 1, 4), device) and _as(norm, f32, (128,), device)
             and _as(input_norm, f32, (h,), device) and _as(post_norm, f32, (h,), device)
@@ -233,6 +239,45 @@ def gdn_commit(state: torch.Tensor, keys: torch.Tensor, u: torch.Tensor, cum: to
               accepted, _ptr(out), _ptr(window), window.shape[2], first, window.shape[1], _ptr(history),
               _stream(device))
     return out, history
+
+
+def attention_mixer_fits(hidden: torch.Tensor, keys: torch.Tensor, values: torch.Tensor, position: int, *,
+                         in_proj: PackedW4, out_proj: PackedW4, input_norm: torch.Tensor, post_norm: torch.Tensor,
+                         q_norm: torch.Tensor, k_norm: torch.Tensor, inv_freq: torch.Tensor, heads: int,
+                         kv_heads: int, head_dim: int, eps: float) -> bool:
+    """Whether :func:`attention_mixer` takes these arguments: head dim 128 or 256, plain contiguous tensors of the
+    dtypes the target keeps, room in the cache, and no gradient asked for."""
+    if not _residual(hidden) or head_dim not in (128, 256) or keys.ndim != 4 or keys.shape[2] > 1 << 24:
+        return False
+    device, (t, h) = hidden.device, hidden.shape
+    f32, b16, cache, half = torch.float32, torch.bfloat16, (1, kv_heads, keys.shape[2], head_dim), inv_freq.shape[0]
+    return (t * heads <= 1 << 22 and heads <= 1024 and heads % kv_heads == 0 and position + t <= keys.shape[2]
+            and half > 0 and half % (head_dim // 64) == 0 and 2 * half <= head_dim
+            and _as(keys, b16, cache, device) and _as(values, b16, cache, device)
+            and _as(inv_freq, f32, (half,), device)
+            and _as(input_norm, f32, (h,), device) and _as(post_norm, f32, (h,), device)
+            and _as(q_norm, f32, (head_dim,), device) and _as(k_norm, f32, (head_dim,), device)
+            and _matrix(in_proj, 2 * (heads + kv_heads) * head_dim, h, device)
+            and _matrix(out_proj, h, heads * head_dim, device))
+
+
+def attention_mixer(hidden: torch.Tensor, keys: torch.Tensor, values: torch.Tensor, position: int, *,
+                    in_proj: PackedW4, out_proj: PackedW4, input_norm: torch.Tensor, post_norm: torch.Tensor,
+                    q_norm: torch.Tensor, k_norm: torch.Tensor, inv_freq: torch.Tensor, heads: int, kv_heads: int,
+                    head_dim: int, eps: float) -> tuple[torch.Tensor, torch.Tensor]:
+    """An attention layer from its residual to the MoE input, in one call: norm, in_proj, Q/K norms, rotary, cache
+    append, attention, output gate, out_proj, residual add, post-norm.  Returns ``(mid, normed)`` (fp32, bf16
+    ``[T, H]``).  Tensors as :func:`attention_mixer_fits` accepts them."""
+    device, (t, h) = hidden.device, hidden.shape
+    mid = torch.empty((t, h), dtype=torch.float32, device=device)
+    normed = torch.empty((t, h), dtype=torch.bfloat16, device=device)
+    desc = _lib.AttentionDesc(_desc(in_proj), _desc(out_proj), input_norm.data_ptr(), post_norm.data_ptr(),
+                              q_norm.data_ptr(), k_norm.data_ptr(), inv_freq.data_ptr(), h, heads, kv_heads, head_dim,
+                              2 * inv_freq.shape[0], eps)
+    ws = _workspace(_lib.load().dflash_attention_workspace_bytes(t, h, heads, kv_heads, head_dim), device, None)
+    _lib.call("dflash_attention_mixer", ctypes.byref(desc), _ptr(hidden), t, position, _ptr(keys), _ptr(values),
+              keys.shape[2], _ptr(mid), _ptr(normed), _ptr(ws), ws.numel(), _stream(device))
+    return mid, normed
 
 
 def router_logits(hidden: torch.Tensor, router_weight: torch.Tensor) -> torch.Tensor:

@@ -323,20 +323,34 @@ class TargetModel:
                                                      r.u.split(n, 2), r.cum.split(n, 2))]
         return r.mid, r.normed, GdnPending(r.window, state, chunks)
 
+    def _attention_kernels(self, hidden: Tensor, lw: LayerWeights, keys: Tensor, values: Tensor, pos: int):
+        """The mixer half of an attention layer on the HIP kernels: ``(mid, moe input)``, or ``None`` when the
+        layer is not one they take (``ops.attention_mixer_fits``)."""
+        c = self.config
+        args = dict(in_proj=lw.mixer_in, out_proj=lw.mixer_out, input_norm=lw.input_norm, post_norm=lw.post_norm,
+                    q_norm=lw.q_norm, k_norm=lw.k_norm, inv_freq=self.inv_freq, heads=c.heads, kv_heads=c.kv_heads,
+                    head_dim=c.head_dim, eps=c.rms_eps)
+        if not ops.attention_mixer_fits(hidden, keys, values, pos, **args):
+            return None
+        return ops.attention_mixer(hidden, keys, values, pos, **args)
+
     def layer(self, i: int, hidden: Tensor, state: TargetState, workspace: Optional[Tensor] = None,
               trace: Optional[dict] = None):
         """One decoder layer on the fp32 residual ``[T, H]``; returns (hidden, GdnPending or None).
         ``trace`` (a dict) receives the residual after the mixer and the MoE input."""
         c, lw = self.config, self.w.layers[i]
+        pending = None
         if lw.kind == "linear_attention":
             done = self._gdn_kernels(hidden, lw, state.conv[i], state.recurrent[i])
-            if done is not None:
-                mid, normed, pending = done
-                if trace is not None:
-                    trace.update(mid=mid, moe_in=normed)
-                return mid + self._moe(normed, lw, workspace), pending     # bf16 joins the fp32 sum exactly
+        else:
+            done = self._attention_kernels(hidden, lw, state.keys[i], state.values[i], state.position)
+        if done is not None:
+            mid, normed, *rest = done
+            pending = rest[0] if rest else None
+            if trace is not None:
+                trace.update(mid=mid, moe_in=normed)
+            return mid + self._moe(normed, lw, workspace), pending         # bf16 joins the fp32 sum exactly
         normed = layers.rms_normalise(hidden, lw.input_norm, c.rms_eps, 1.0).to(torch.bfloat16)
-        pending = None
         if lw.kind == "linear_attention":
             mixed, pending = self._gdn(normed, lw, state.conv[i], state.recurrent[i])
         else:

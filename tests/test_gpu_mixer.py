@@ -59,3 +59,35 @@ def test_gdn_layer_takes_the_general_path_for_other_forms(pkg, device):
     assert not pkg.ops.gdn_mixer_fits(x, state.conv[0], state.recurrent[0], **model._gdn_args(model.w.layers[0]))
     got, _ = model.layer(0, x, state)
     assert metrics.compare(got.cpu(), want.cpu())["max_rel"] <= TOL
+
+
+@pytest.mark.parametrize("heads,kv_heads,head_dim", [(4, 2, 128), (16, 2, 256)])
+@pytest.mark.parametrize("tokens,context", [(1, 0), (1, 1), (1, 300), (2, 31), (15, 113), (16, 0), (16, 1000), (17, 40),
+                                            (32, 97), (37, 0), (130, 5)])
+def test_attention_layer_matches_oracle(pkg, device, tokens, context, heads, kv_heads, head_dim):
+    """Lengths around the kernels' edges: row tiles of 16 (a token has heads / kv_heads rows), 32 keys a wave, 128 keys a
+    workgroup, one split and many, splits past a tile's last key.  Output and K rows within one bf16 ulp (above)."""
+    base = pkg.target.small_config(("full_attention",))
+    c = type(base)(**{**vars(base), "heads": heads, "kv_heads": kv_heads, "head_dim": head_dim})
+    host = pkg.target.random_weights(c, seed=9, device="cpu", layout="portable", generate_on="cpu")
+    layout = "tiled" if tokens <= 32 else "portable"
+    model = pkg.target.TargetModel(pkg.target.to_device(host, device, layout=layout), capacity=context + tokens + 3)
+    state = model.synthetic_context(context, seed=10)
+    state.keys[0].mul_(4.0)                         # scores of several units, so that the softmax is not flat
+    before = oracle_layer_state(state, 0)
+    untouched = state.keys[0][:, :, context + tokens:].clone()
+    x = torch.randn((tokens, c.hidden), generator=torch.Generator().manual_seed(tokens + context))
+    trace = {}
+    out, pending = model.layer(0, x.to(device), state, trace=trace)
+    assert pending is None and trace["mid"].dtype == torch.float32
+    lw = oracle_layer_weights(host.layers[0])
+    normed = stack.bf16(stack.norm(x, lw["input_norm"], c.rms_eps, 1.0))
+    ref = stack.attention_layer(normed, lw, before["keys"], before["values"], context, c)
+    mixer = trace["mid"].cpu() - x                  # the residual would hide it
+    print(f"attention T={tokens} ctx={context} D={head_dim}", metrics.compare(mixer, ref["out"]), flush=True)
+    assert metrics.compare(mixer, ref["out"])["max_rel"] <= TOL
+    rows = slice(context, context + tokens)
+    assert metrics.compare(state.keys[0][0, :, rows].float().cpu(), ref["keys"])["max_rel"] <= TOL
+    assert metrics.compare(state.values[0][0, :, rows].float().cpu(), ref["values"])["max_rel"] <= TOL
+    assert torch.equal(state.keys[0][:, :, context + tokens:], untouched)
+    assert torch.equal(state.keys[0][0, :, :context].cpu(), before["keys"][:, :context])
