@@ -678,9 +678,10 @@ const char* dflash_last_error(void) { return g_last_error.c_str(); }
 
 size_t dflash_qlinear_workspace_bytes(int64_t m, int64_t k, int64_t group_size) {
   if (m < 0 || k <= 0 || group_size <= 0) return 0;
+  const size_t rows = (static_cast<size_t>(m) + 31) / 32 * 32;
   Carver c;
-  c.take(2 * static_cast<size_t>(m) * k);
-  c.take(4 * static_cast<size_t>(m) * (k / 128));
+  c.take(2 * rows * k);
+  c.take(4 * rows * (k / 128));
   return c.off;
 }
 
@@ -735,46 +736,30 @@ int qlinear_impl(const void* x, int64_t m, const dflash_w4* weight, void* y, boo
       else dflash::launch_w4_small(sp, st);
       return launch_status("qlinear");
     }
-    // GEMM kernel: verify (m <= 32), else the streaming kernel (or its per-wave fallback)
+    // the verify kernel for the wide outputs of up to 32 rows, else w4_linear
     dflash::VerifyParams vl{};
     // the verify kernel stages at most 16 rows of K = 4096; 17..32 rows run as two launches of it
     const int64_t vrows = K == 4096 && m > 16 && m <= 32 ? 16 : m;
     const bool verify = (weight->group_size == 128 || weight->group_size == 256) &&
                         dflash::verify_layout(dflash::kModeLinear, static_cast<int>(vrows), static_cast<int>(K),
                                               static_cast<int>(N), 1, 1, 0, 0, &vl);
+    // tiled banks are taken in the shapes the contract names (group 128, K of 512, 1024 or 2048, N a multiple of
+    // 32 times the row groups above 32 rows), not in all that the kernel could read
     if (tiled && !verify &&
         !w4_path_reads_tiled(dflash::kModeLinear, static_cast<int>(N), static_cast<int>(K),
                              static_cast<int>(weight->group_size), GemmPath::kStream))
       return tiled_unsupported("qlinear");
-    Carver c;
-    uint16_t* x_il = at<uint16_t>(workspace, c.take(2 * static_cast<size_t>(m) * K));
-    float* xneg = at<float>(workspace, c.take(4 * static_cast<size_t>(m) * (K / 128)));
-    if (!verify) {  // the verify kernel converts the raw rows itself
-      dflash::FrontParams f{};
-      f.x = static_cast<const uint16_t*>(x);
-      f.T = static_cast<int>(m);
-      f.prep_rows = static_cast<int>(m);
-      f.H = static_cast<int>(K);
-      f.x_il = x_il;
-      f.xneg = xneg;
-      dflash::launch_front(f, st);
-      if (int r = launch_status("prep")) return r;
-    }
-    dflash::W4StreamParams p{};
-    p.w = static_cast<const uint8_t*>(weight->packed);
-    p.s = weight->scales;
-    p.tiled = weight->layout == DFLASH_LAYOUT_TILED ? 1 : 0;
-    p.N = static_cast<int>(N);
-    p.K = static_cast<int>(K);
-    p.G = static_cast<int>(weight->group_size);
-    p.act = x_il;
-    p.act_neg = xneg;
-    p.neg_parts = 1;
-    p.out_bf16 = y_f32 ? nullptr : static_cast<uint16_t*>(y);
-    p.out_f32 = y_f32 ? static_cast<float*>(y) : nullptr;
-    p.M = static_cast<int>(m);
     if (verify) {
-      p.act_neg = nullptr;
+      dflash::W4StreamParams p{};
+      p.w = static_cast<const uint8_t*>(weight->packed);
+      p.s = weight->scales;
+      p.tiled = tiled ? 1 : 0;
+      p.N = static_cast<int>(N);
+      p.K = static_cast<int>(K);
+      p.G = static_cast<int>(weight->group_size);
+      p.neg_parts = 1;
+      p.out_bf16 = y_f32 ? nullptr : static_cast<uint16_t*>(y);
+      p.out_f32 = y_f32 ? static_cast<float*>(y) : nullptr;
       p.rows_per_pass = 16;
       p.strips = p.N / 32;
       for (int64_t r0 = 0; r0 < m; r0 += vrows) {
@@ -788,10 +773,24 @@ int qlinear_impl(const void* x, int64_t m, const dflash_w4* weight, void* y, boo
       }
       return DFLASH_OK;
     }
-    const int mt = token_tiles(m);
-    p.rows_per_pass = 16 * mt;
-    launch_w4(dflash::kModeLinear, weight->scale_dtype == DFLASH_DTYPE_F32, mt, 1, GemmPath::kStream,
-              p, st);
+    if (!dflash::w4_linear_fits(m, N, K)) return fail(DFLASH_ERR_UNSUPPORTED, "qlinear: K must stay below 2^25");
+    const size_t rows = (static_cast<size_t>(m) + 31) / 32 * 32;
+    Carver c;
+    dflash::LinearParams lp{};
+    lp.x = static_cast<const uint16_t*>(x);
+    lp.w = static_cast<const uint8_t*>(weight->packed);
+    lp.s = weight->scales;
+    lp.y = y;
+    lp.xf = at<uint16_t>(workspace, c.take(2 * rows * K));
+    lp.neg = at<float>(workspace, c.take(4 * rows * (K / 128)));
+    lp.M = static_cast<int>(m);
+    lp.N = static_cast<int>(N);
+    lp.K = static_cast<int>(K);
+    lp.G = static_cast<int>(weight->group_size);
+    lp.tiled = tiled ? 1 : 0;
+    lp.scale_f32 = weight->scale_dtype == DFLASH_DTYPE_F32 ? 1 : 0;
+    lp.y_f32 = y_f32 ? 1 : 0;
+    dflash::launch_w4_linear(lp, cu_count(), st);
     return launch_status("qlinear");
   } catch (...) {
     return fail(DFLASH_ERR_HIP, "unexpected host exception");

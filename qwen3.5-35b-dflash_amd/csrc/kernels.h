@@ -106,9 +106,9 @@ __device__ __forceinline__ void write_slot(int4* slot_table, int32_t* pass_slot,
 
 enum W4Mode : int { kModeLinear = 0, kModeGateUp = 1, kModeDown = 2 };
 
-// Persistent streaming W4A16 GEMM over the routing work table (w4_stream.hip).
+// Persistent streaming W4A16 GEMM over the routing work table (w4_stream.hip); kModeLinear: the verify kernel only.
 struct W4StreamParams {
-  const uint8_t* w;        // packed int4 [E][N][K/2] (or [N][K/2] for kModeLinear)
+  const uint8_t* w;        // packed int4 [E][N][K/2] (one matrix for kModeLinear)
   const void* s;           // scales [E][N][K/G], bf16 or fp32
   const uint8_t* w_shared; // shared-expert packed [N][K/2] or null
   const void* s_shared;
@@ -275,6 +275,20 @@ void launch_w4_small(const SmallLinearParams& p, hipStream_t stream);
 // its streaming form (persistent workgroups, x in registers): M <= 16
 bool small_linear_stream_fits(int M, int N, int K, int G);
 void launch_w4_small_stream(const SmallLinearParams& p, int grid, hipStream_t stream);
+
+// The linear for any row count (w4_linear.hip): K % 128 == 0, N % 32 == 0, G in {128, 256}.
+struct LinearParams {
+  const uint16_t* x;       // bf16 [M][K]
+  const uint8_t* w;        // packed int4 [N][K/2], portable or tiled
+  const void* s;           // scales [N][K/G] (tiled: [N/16][K/G][16]), bf16 or fp32
+  void* y;                 // [M][N], bf16 or fp32
+  uint16_t* xf;            // scratch: x in fragment order, [ceil(M/32)][K/128][8][64 lanes][8]
+  float* neg;              // scratch: offset terms, [ceil(M/32)][K/128][32]
+  int M, N, K, G;
+  int tiled, scale_f32, y_f32;
+};
+bool w4_linear_fits(int64_t M, int64_t N, int64_t K);
+void launch_w4_linear(const LinearParams& p, int cus, hipStream_t stream);
 
 // Gated-DeltaNet mixer around its projections (gdn.hip): head dims 128, four conv taps.
 constexpr int kMaxNormWidth = 8192;  // row width launch_add_norm takes (a multiple of 4)

@@ -11,7 +11,6 @@
 // tot += (-136*sum_group x) x scale.
 //
 // Semantics per mode (reference citations):
-//   kModeLinear : y = x . dequant(W)^T, bf16 out                 (fused/quantization.py:154-165)
 //   kModeGateUp : h = silu(x.Wg^T) * (x.Wu^T), gate rows first   (reference/fused_ops.py:170-171,
 //                 h rounded to bf16, stored octet-interleaved      fused/quantization.py:193-195)
 //   kModeDown   : y = route_weight * (h . Wd^T), fp32 out        (fused/quantization.py:196-199)
@@ -32,8 +31,7 @@ __device__ __forceinline__ void w4_pass(const W4StreamParams& p, const uint8_t* 
   for (int mt = 0; mt < kMT; ++mt) {
     const int m = min(m0 + mt * 16 + lr, M - 1);
     if (kMode == kModeGateUp) arow[mt] = shared ? m : p.tok[seg + m];
-    else if (kMode == kModeDown) arow[mt] = shared ? p.T * p.top_k + m : seg + m;
-    else arow[mt] = m;
+    else arow[mt] = shared ? p.T * p.top_k + m : seg + m;
   }
   const uint16_t* ap[kMT];
 #pragma unroll
@@ -119,17 +117,7 @@ __device__ __forceinline__ void w4_pass(const W4StreamParams& p, const uint8_t* 
     for (int e = 0; e < 4; ++e) {
       const int m = m0 + mt * 16 + 4 * kq + e;
       const bool valid = m < M;
-      if (kMode == kModeLinear) {
-        if (valid && p.out_f32) {  // fp32 output: the unrounded sums
-          float* o = p.out_f32 + static_cast<int64_t>(m) * p.N;
-          o[row0 + lr] = tot0[mt][e];
-          o[row1 + lr] = tot1[mt][e];
-        } else if (valid) {
-          uint16_t* o = p.out_bf16 + static_cast<int64_t>(m) * p.N;
-          o[row0 + lr] = f32_to_bf16(tot0[mt][e]);
-          o[row1 + lr] = f32_to_bf16(tot1[mt][e]);
-        }
-      } else if (kMode == kModeGateUp) {
+      if (kMode == kModeGateUp) {
         const int inter = p.N >> 1;
         const int col = strip * 16 + lr;
         const uint16_t hb = f32_to_bf16(silu(tot0[mt][e]) * tot1[mt][e]);
@@ -152,32 +140,23 @@ __device__ __forceinline__ void w4_pass(const W4StreamParams& p, const uint8_t* 
 
 template <int kMode, typename ScaleT>
 __global__ __launch_bounds__(256) void w4_gemm_kernel(W4StreamParams p, int max_slots) {
-  const int items_per_slot = p.N >> 5;  // gate_up: I/16 column pairs; down, linear: 32-row strips
+  const int items_per_slot = p.N >> 5;  // gate_up: I/16 column pairs; down: 32-row strips
   const int item = blockIdx.x * 4 + (threadIdx.x >> 6);
   const int slot = item / items_per_slot;
   const int strip = item - slot * items_per_slot;
   if (slot >= max_slots) return;
   const uint8_t* w;
   const ScaleT* s;
-  int seg = 0, M;
-  bool shared = false;
-  if (kMode == kModeLinear) {
-    w = p.w;
-    s = static_cast<const ScaleT*>(p.s);
-    M = p.M;
+  if (slot >= p.meta[0] + p.has_shared) return;
+  const int4 d = p.slot_table[slot];  // expert (-1 shared), segment start, rows, first pass
+  const int seg = d.y, M = d.z;
+  const bool shared = d.x < 0;
+  if (shared) {
+    w = p.w_shared;
+    s = static_cast<const ScaleT*>(p.s_shared);
   } else {
-    if (slot >= p.meta[0] + p.has_shared) return;
-    const int4 d = p.slot_table[slot];  // expert (-1 shared), segment start, rows, first pass
-    seg = d.y;
-    M = d.z;
-    if (d.x < 0) {
-      shared = true;
-      w = p.w_shared;
-      s = static_cast<const ScaleT*>(p.s_shared);
-    } else {
-      w = p.w + d.x * p.w_stride;
-      s = static_cast<const ScaleT*>(p.s) + d.x * p.s_stride;
-    }
+    w = p.w + d.x * p.w_stride;
+    s = static_cast<const ScaleT*>(p.s) + d.x * p.s_stride;
   }
   int row0, row1;
   if (kMode == kModeGateUp) {
@@ -206,7 +185,6 @@ void launch_w4_gemm(int mode, bool fp32_scales, int max_slots, const W4StreamPar
   if (fp32_scales) hipLaunchKernelGGL((w4_gemm_kernel<MODE, float>), grid, block, 0, stream, p, max_slots); \
   else hipLaunchKernelGGL((w4_gemm_kernel<MODE, uint16_t>), grid, block, 0, stream, p, max_slots);
   switch (mode) {
-    case kModeLinear: DFLASH_W4_LAUNCH(kModeLinear) break;
     case kModeGateUp: DFLASH_W4_LAUNCH(kModeGateUp) break;
     default: DFLASH_W4_LAUNCH(kModeDown) break;
   }

@@ -25,7 +25,6 @@
 // range) so the in-order vmcnt accounting keeps all newer buffers in flight.
 //
 // Modes:
-//   kModeLinear : y = x . dequant(W)^T, bf16 out                 (fused/quantization.py:154-165)
 //   kModeGateUp : h = silu(x.Wg^T) * (x.Wu^T), bf16, interleaved   (reference/fused_ops.py:170-171)
 //   kModeDown   : y = route_weight * (h . Wd^T), fp32             (fused/quantization.py:196-199)
 #include "kernels.h"
@@ -80,17 +79,9 @@ struct SlotDesc {
   int e, seg, M, pass0, pass_end;
 };
 
-template <int kMode, int kMT>
-__device__ __forceinline__ SlotDesc load_slot(const W4StreamParams& p, int slot, int total_passes) {
+template <int kMT>
+__device__ __forceinline__ SlotDesc load_slot(const W4StreamParams& p, int slot) {
   SlotDesc d;
-  if (kMode == kModeLinear) {
-    d.e = 0;
-    d.seg = 0;
-    d.M = p.M;
-    d.pass0 = 0;
-    d.pass_end = total_passes;
-    return d;
-  }
   const int4 v = ld_const_int4(p.slot_table, slot);
   d.e = v.x;
   d.seg = v.y;
@@ -216,7 +207,7 @@ __global__ __launch_bounds__(512) void w4_stream_kernel(W4StreamParams p) {
   const int S = nkb / kKBPW, RG = 8 / S;  // S in {4, 8}: one k-split wave per output phase e < 4
   const int rg = wave / S, ks = wave - rg * S;
 
-  const int total_passes = kMode == kModeLinear ? (p.M + 16 * kMT - 1) / (16 * kMT) : ld_const(p.meta, 1);
+  const int total_passes = ld_const(p.meta, 1);
   const int64_t total_units = static_cast<int64_t>(total_passes) * p.strips;
   const int u_begin = static_cast<int>(total_units * blockIdx.x / gridDim.x);
   const int u_end = static_cast<int>(total_units * (blockIdx.x + 1) / gridDim.x);
@@ -244,13 +235,13 @@ __global__ __launch_bounds__(512) void w4_stream_kernel(W4StreamParams p) {
   // ---- load stream: uniform cursor and row pointers (tile 0 of the wave's row group)
   int l_u = u_begin;
   int l_P = l_u / p.strips, l_strip = l_u - l_P * p.strips;
-  int l_slot = kMode == kModeLinear ? 0 : ld_const(p.pass_slot, l_P);
-  SlotDesc ld = load_slot<kMode, kMT>(p, l_slot, total_passes);
+  int l_slot = ld_const(p.pass_slot, l_P);
+  SlotDesc ld = load_slot<kMT>(p, l_slot);
   const uint8_t* l_w;  // weights of the current unit
   const uint8_t* l_s;  // scales of the current unit (bytes)
   auto slot_bases = [&](const SlotDesc& d) {
-    const bool shared = kMode != kModeLinear && d.e < 0;
-    const int64_t e = kMode == kModeLinear ? 0 : d.e;
+    const bool shared = d.e < 0;
+    const int64_t e = d.e;
     l_w = (shared ? p.w_shared : p.w + e * p.w_stride) + w_first;
     l_s = static_cast<const uint8_t*>(shared ? p.s_shared : static_cast<const void*>(static_cast<const ScaleT*>(p.s) + e * p.s_stride)) +
           s_first * static_cast<int64_t>(sizeof(ScaleT));
@@ -275,7 +266,7 @@ __global__ __launch_bounds__(512) void w4_stream_kernel(W4StreamParams p) {
       if (++l_strip == p.strips) {
         l_strip = 0;
         ++l_P;
-        if (kMode != kModeLinear && l_P == ld.pass_end) ld = load_slot<kMode, kMT>(p, ++l_slot, total_passes);
+        if (l_P == ld.pass_end) ld = load_slot<kMT>(p, ++l_slot);
         slot_bases(ld);
       }
     }
@@ -287,8 +278,8 @@ __global__ __launch_bounds__(512) void w4_stream_kernel(W4StreamParams p) {
 
   // ---- compute stream
   int c_P = u_begin / p.strips, c_strip = u_begin - c_P * p.strips;
-  int c_slot = kMode == kModeLinear ? 0 : ld_const(p.pass_slot, c_P);
-  SlotDesc cd = load_slot<kMode, kMT>(p, c_slot, total_passes);
+  int c_slot = ld_const(p.pass_slot, c_P);
+  SlotDesc cd = load_slot<kMT>(p, c_slot);
   ActRegs<kMT, kKBPW> A;
   int act_pass = -1, m0 = 0, buf = 0;
   const int inter = p.N >> 1;
@@ -309,7 +300,7 @@ __global__ __launch_bounds__(512) void w4_stream_kernel(W4StreamParams p) {
     if (live) {
       const int colblock = c_strip * RG + rg;
       const int row0 = colblock * kTileRows;
-      const bool shared = kMode != kModeLinear && cd.e < 0;
+      const bool shared = cd.e < 0;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         if (e != ks) continue;
@@ -324,17 +315,7 @@ __global__ __launch_bounds__(512) void w4_stream_kernel(W4StreamParams p) {
           }
           const int m = m0 + mt * 16 + 4 * kq + e;
           const bool valid = m < cd.M;
-          if (kMode == kModeLinear) {
-            if (valid && p.out_f32) {  // fp32 output: the unrounded sums
-              float* o = p.out_f32 + static_cast<int64_t>(m) * p.N + row0 + lr;
-              o[0] = v0;
-              o[second] = v1;
-            } else if (valid) {
-              uint16_t* o = p.out_bf16 + static_cast<int64_t>(m) * p.N + row0 + lr;
-              o[0] = f32_to_bf16(v0);
-              o[second] = f32_to_bf16(v1);
-            }
-          } else if (kMode == kModeGateUp) {
+          if (kMode == kModeGateUp) {
             const uint16_t hb = f32_to_bf16(silu(v0) * v1);
             const int hrow = shared ? p.T * p.top_k + m : cd.seg + m;
             if (valid) p.out_bf16[static_cast<int64_t>(hrow) * inter + octet_slot(row0 + lr)] = hb;
@@ -356,8 +337,8 @@ __global__ __launch_bounds__(512) void w4_stream_kernel(W4StreamParams p) {
       if (++c_strip == p.strips) {
         c_strip = 0;
         ++c_P;
-        if (kMode != kModeLinear && c_P == cd.pass_end && c_P < total_passes)
-          cd = load_slot<kMode, kMT>(p, ++c_slot, total_passes);
+        if (c_P == cd.pass_end && c_P < total_passes)
+          cd = load_slot<kMT>(p, ++c_slot);
       }
     }
     buf ^= 1;
@@ -390,7 +371,6 @@ void launch_w4_stream(int mode, bool fp32_scales, int mt, int grid, const W4Stre
   if (mt == 1) { DFLASH_STREAM_KB(MODE, 1) }  \
   else { DFLASH_STREAM_KB(MODE, 2) }
   switch (mode) {
-    case kModeLinear: DFLASH_STREAM_MT(kModeLinear) break;
     case kModeGateUp: DFLASH_STREAM_MT(kModeGateUp) break;
     default: DFLASH_STREAM_MT(kModeDown) break;
   }
