@@ -14,7 +14,8 @@
 // spans few tokens.
 //
 // Bound by latency at verify sizes (T = 16 behind 4001 keys, 16 heads over 2 KV heads of 256: 8.4 MB of cache, 1.7 us at
-// the copy rate): prep 4.8, split 18.4, combine 10.0 us, in place of 60 library launches (250 us).  Against 64
+// the copy rate): prep 4.5, split 15.3 (19.0 with the row tiles of a split spread over the XCDs), combine 4.8 (9.8 with the
+// splits read one after the other), in place of 60 library launches (250 us).  Against 64
 // bits the attention output is 4e-7 to 7e-7 off (fp32 library products 4e-7 to 1.8e-6).
 #include <algorithm>
 
@@ -114,7 +115,9 @@ __global__ __launch_bounds__(256, 1) void attn_split_kernel(AttnParams p) {
   constexpr int kPitch = D + 4;
   __shared__ __align__(16) float osum[4][16][kPitch];
   __shared__ float mx[4][16], ls[4][16];
-  const int tile = blockIdx.x, split = blockIdx.y, kvh = blockIdx.z;
+  // splits fastest: with a multiple of eight of them (workgroups go round robin over the XCDs) a split's keys and values
+  // pass through one XCD's L2 only, for all row tiles
+  const int tile = blockIdx.x / p.splits, split = blockIdx.x - tile * p.splits, kvh = blockIdx.z;
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int lr = lane & 15, kq = lane >> 4;
   const int group = p.heads / p.kv, rows = p.T * group;
@@ -247,24 +250,46 @@ __global__ __launch_bounds__(256, 1) void attn_split_kernel(AttnParams p) {
   }
 }
 
-// One workgroup per (token, head), one dim a thread; splits that hold no key of the row are skipped.
+// One workgroup per (token, head), one dim a thread.  Each wave reads every split's maximum and sum at once, a split a
+// lane (one after the other they were most of this kernel's time), and the partial rows follow eight at a time.  Splits
+// that hold no key of the row (maximum -inf, partial row never written) are left out.
+constexpr int kMaxSplits = 256;
 template <int D>
 __global__ __launch_bounds__(D) void attn_combine_kernel(AttnParams p) {
-  const int t = blockIdx.x / p.heads, head = blockIdx.x - t * p.heads, c = threadIdx.x;
+  __shared__ float fs[kMaxSplits];
+  const int t = blockIdx.x / p.heads, head = blockIdx.x - t * p.heads, c = threadIdx.x, lane = threadIdx.x & 63;
   const int group = p.heads / p.kv, rows = p.T * group;
   const int64_t row = static_cast<int64_t>(head / group) * rows + t * group + head % group;
   const int64_t stride = static_cast<int64_t>(p.kv) * rows;
   const float gate = bf16_to_f32(p.proj[static_cast<int64_t>(t) * p.ldp + head * 2 * D + D + c]);
-  float M = -__builtin_inff();
-  for (int s = 0; s < p.splits; ++s) M = fmaxf(M, p.ml[s * stride + row].x);
-  float l = 0.f, o = 0.f;
-#pragma unroll 4
-  for (int s = 0; s < p.splits; ++s) {
-    const float2 v = p.ml[s * stride + row];
-    if (v.x == -__builtin_inff()) continue;
-    const float f = expf(v.x - M);
-    l += v.y * f;
-    o += p.part[(s * stride + row) * D + c] * f;
+  constexpr int kPer = kMaxSplits / 64;
+  float2 v[kPer];
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) {
+    const int s = lane + 64 * i;
+    v[i] = s < p.splits ? p.ml[s * stride + row] : make_float2(-__builtin_inff(), 0.f);
+  }
+  float M = fmaxf(fmaxf(v[0].x, v[1].x), fmaxf(v[2].x, v[3].x));
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) M = fmaxf(M, __shfl_xor(M, o, 64));
+  float l = 0.f;
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) {
+    const bool used = v[i].x != -__builtin_inff();
+    const float f = used ? expf(v[i].x - M) : -1.f;
+    if (used) l += v[i].y * f;
+    if (threadIdx.x < 64) fs[lane + 64 * i] = f;
+  }
+  l = wave_sum(l);
+  __syncthreads();
+  float o = 0.f;
+  for (int s0 = 0; s0 < p.splits; s0 += 8) {
+    float x[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) x[i] = p.part[(min(s0 + i, p.splits - 1) * stride + row) * D + c];
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      if (s0 + i < p.splits && fs[s0 + i] >= 0.f) o += x[i] * fs[s0 + i];
   }
   p.out[(static_cast<int64_t>(t) * p.heads + head) * D + c] = f32_to_bf16(o / l / (1.0f + expf(-gate)));
 }
@@ -275,7 +300,7 @@ __global__ __launch_bounds__(D) void attn_combine_kernel(AttnParams p) {
 // only add partial rows (splits * rows * D * 4 bytes, written and read again).
 int attn_splits(int rows, int kv, int keys, int cus) {
   const int tiles = kv * ((rows + 15) / 16);
-  return std::max(1, std::min((keys + 127) / 128, cus / tiles));
+  return std::max(1, std::min({(keys + 127) / 128, cus / tiles, kMaxSplits}));
 }
 int64_t attn_partial_rows(int rows, int kv, int cus) {
   // splits <= max(1, cus / tiles), and a tile holds 16 rows
@@ -286,7 +311,7 @@ template <int D>
 static void launch_attn(const AttnParams& p, hipStream_t stream) {
   const int rows = p.T * (p.heads / p.kv);
   hipLaunchKernelGGL(attn_prep_kernel<D>, dim3((p.T * (p.heads + 2 * p.kv) + 3) / 4), dim3(256), 0, stream, p);
-  hipLaunchKernelGGL(attn_split_kernel<D>, dim3((rows + 15) / 16, p.splits, p.kv), dim3(256), 0, stream, p);
+  hipLaunchKernelGGL(attn_split_kernel<D>, dim3((rows + 15) / 16 * p.splits, 1, p.kv), dim3(256), 0, stream, p);
   hipLaunchKernelGGL(attn_combine_kernel<D>, dim3(p.T * p.heads), dim3(D), 0, stream, p);
 }
 void launch_attention(int head_dim, const AttnParams& p, hipStream_t stream) {
