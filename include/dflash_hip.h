@@ -215,6 +215,19 @@ int dflash_moe_split_down(int64_t tokens, int64_t hidden_size, int64_t inter_siz
                           int64_t group_size, int has_shared, int32_t scale_dtype, int32_t layout);
 
 /*
+ * dflash_moe_w4a16 with the residual add that follows it in a decoder layer
+ * (model/qwen35_moe_dflash/fused/model.py:305-307): sum = residual + (the layer's bf16 output), fp32
+ * [tokens][hidden_size].  sum may be residual itself.  Other arguments, constraints and workspace as there; the
+ * router always runs.
+ */
+int dflash_moe_w4a16_residual(const void* hidden, int64_t tokens, int64_t hidden_size, const void* router_weight,
+                              int64_t top_k, const dflash_w4* gate_up, const dflash_w4* down,
+                              const dflash_w4* shared_gate_up, const dflash_w4* shared_down,
+                              const void* shared_gate_weight, const float* residual, float* sum, float* logits_out,
+                              int32_t* topk_ids, float* topk_weights, int32_t* perm, int32_t* inv_perm,
+                              int32_t* expert_offsets, void* workspace, size_t workspace_bytes, void* stream);
+
+/*
  * dflash_moe_w4a16 without a workspace: the same layer, arguments and results, with its
  * scratch in a static device array of DFLASH_NOALLOC_SCRATCH_BYTES (8 MiB) that each GPU
  * the library runs on holds until the process ends.  No counterpart in the reference: it

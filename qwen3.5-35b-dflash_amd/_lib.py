@@ -109,6 +109,8 @@ SIGNATURES = {
                                                 _P, _P, _P, _SZ, _P]),
     "dflash_moe_w4a16": (ctypes.c_int, [_P, _I64, _I64, _P, _P, _I64, _W4P, _W4P, _W4P, _W4P, _P, _P, _P, _P, _P,
                                         _P, _P, _P, _P, _SZ, _P]),
+    "dflash_moe_w4a16_residual": (ctypes.c_int, [_P, _I64, _I64, _P, _I64, _W4P, _W4P, _W4P, _W4P, _P, _P, _P, _P, _P,
+                                                 _P, _P, _P, _P, _P, _SZ, _P]),
     "dflash_moe_w4a16_noalloc": (ctypes.c_int, [_P, _I64, _I64, _P, _P, _I64, _W4P, _W4P, _W4P, _W4P, _P, _P, _P, _P,
                                                 _P, _P, _P, _P, _P]),
     "dflash_gdn_workspace_bytes": (_SZ, [_I64, _I64, _I64, _I64]),

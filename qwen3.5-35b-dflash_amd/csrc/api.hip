@@ -211,6 +211,8 @@ struct MoeShapes {
   bool gu_f32, dn_f32;
   bool scales16;  // every scale bank 16-byte aligned (row scales load as 16-byte words)
   bool tiled;     // every bank in the tiled layout
+  const float* residual = nullptr;  // with sum: the layer leaves residual + output there in fp32
+  float* sum = nullptr;
 };
 
 // Long prefill (at least 16 rows per expert on average) runs both expert GEMMs
@@ -477,14 +479,15 @@ int run_verify(const MoeShapes& S, dflash::VerifyParams gu, dflash::VerifyParams
   }
 
   if (measuring()) return DFLASH_OK;
+  const CombineOut combined{static_cast<uint16_t*>(out), S.residual, S.sum};
   if (fused) {
     launch_combine_parts(at<float>(ws, L.ypart), at<int2>(ws, L.row_seg), gu.part_rps, inv, T, p.top_k, H,
-                         p.has_shared, wts, at<float>(ws, L.gate), static_cast<uint16_t*>(out), stream);
+                         p.has_shared, wts, at<float>(ws, L.gate), combined, stream);
     return launch_status("combine");
   }
   // the verify down launch leaves y unweighted: the combine applies the routing weights
   launch_combine(at<float>(ws, L.y), inv, T, p.top_k, H, p.has_shared, wts, at<float>(ws, L.gate),
-                 static_cast<uint16_t*>(out), stream);
+                 combined, stream);
   return launch_status("combine");
 }
 
@@ -571,11 +574,11 @@ int run_experts(const MoeShapes& S, const int32_t* inv, void* ws, const MoeLayou
   if (int r = launch_status("down")) return r;
 
   if (measuring()) return DFLASH_OK;
+  const CombineOut combined{static_cast<uint16_t*>(out), S.residual, S.sum};
   if (path == GemmPath::kTile)
-    launch_combine_bf16(at<uint16_t>(ws, L.y), inv, T, k, H, p.has_shared, static_cast<uint16_t*>(out), stream);
+    launch_combine_bf16(at<uint16_t>(ws, L.y), inv, T, k, H, p.has_shared, combined, stream);
   else
-    launch_combine(at<float>(ws, L.y), inv, T, k, H, p.has_shared, nullptr, nullptr, static_cast<uint16_t*>(out),
-                   stream);
+    launch_combine(at<float>(ws, L.y), inv, T, k, H, p.has_shared, nullptr, nullptr, combined, stream);
   return launch_status("combine");
 }
 
@@ -1150,12 +1153,15 @@ static int moe_w4a16_body(const void* hidden, int64_t tokens, int64_t hidden_siz
                           const dflash_w4* shared_gate_up, const dflash_w4* shared_down,
                           const void* shared_gate_weight, void* out, float* logits_out, int32_t* topk_ids,
                           float* topk_weights, int32_t* perm, int32_t* inv_perm, int32_t* expert_offsets,
-                          void* workspace, size_t workspace_bytes, bool static_scratch, void* stream) {
+                          void* workspace, size_t workspace_bytes, bool static_scratch, void* stream,
+                          const float* residual = nullptr, float* sum = nullptr) {
   try {
     MoeShapes S;
     if (int r = check_moe(hidden, tokens, hidden_size, top_k, gate_up, down, shared_gate_up, shared_down,
-                          shared_gate_weight, out, &S))
+                          shared_gate_weight, sum ? sum : out, &S))
       return r;
+    S.residual = residual;
+    S.sum = sum;
     if (!router_logits && !router_weight)
       return fail(DFLASH_ERR_INVALID_ARGUMENT, "either router_logits or router_weight is required");
     if (!router_logits && !aligned16(router_weight))
@@ -1247,6 +1253,19 @@ int dflash_moe_w4a16(const void* hidden, int64_t tokens, int64_t hidden_size, co
   return moe_w4a16_body(hidden, tokens, hidden_size, router_logits, router_weight, top_k, gate_up, down,
                         shared_gate_up, shared_down, shared_gate_weight, out, logits_out, topk_ids, topk_weights,
                         perm, inv_perm, expert_offsets, workspace, workspace_bytes, false, stream);
+}
+
+int dflash_moe_w4a16_residual(const void* hidden, int64_t tokens, int64_t hidden_size, const void* router_weight,
+                              int64_t top_k, const dflash_w4* gate_up, const dflash_w4* down,
+                              const dflash_w4* shared_gate_up, const dflash_w4* shared_down,
+                              const void* shared_gate_weight, const float* residual, float* sum, float* logits_out,
+                              int32_t* topk_ids, float* topk_weights, int32_t* perm, int32_t* inv_perm,
+                              int32_t* expert_offsets, void* workspace, size_t workspace_bytes, void* stream) {
+  if (!residual || !sum || !aligned16(residual) || !aligned16(sum))
+    return fail(DFLASH_ERR_INVALID_ARGUMENT, "moe_residual: residual and sum NULL or not 16-byte aligned");
+  return moe_w4a16_body(hidden, tokens, hidden_size, nullptr, router_weight, top_k, gate_up, down, shared_gate_up,
+                        shared_down, shared_gate_weight, nullptr, logits_out, topk_ids, topk_weights, perm, inv_perm,
+                        expert_offsets, workspace, workspace_bytes, false, stream, residual, sum);
 }
 
 int dflash_moe_w4a16_noalloc(const void* hidden, int64_t tokens, int64_t hidden_size, const float* router_logits,

@@ -161,12 +161,20 @@ __host__ __device__ inline int route_slot_pitch(int T) { return (T + 15) & ~15; 
 int64_t route_zero_words(int T, int E);
 void launch_route(const RouteParams& p, bool zeroed, hipStream_t stream);
 void launch_table_prep(const TableParams& p, hipStream_t stream);
+// Where a combine leaves the layer's rows: bf16, or (sum set) residual + bf16 row in fp32.  A decoder layer's
+// second residual add costs no launch of its own that way (one token: 41 us as an elementwise launch of one
+// workgroup between the layer's own, 4 us at 16 tokens).
+struct CombineOut {
+  uint16_t* bf16;
+  const float* residual;
+  float* sum;
+};
 // out = bf16(sum over slots of y rows): rows pre-weighted when wts is null, else weighted
 // here by wts [T*k] (flat pair order) and gate [T] (shared expert).
 void launch_combine(const float* y, const int32_t* inv, int T, int k, int H, int has_shared, const float* wts,
-                    const float* gate, uint16_t* out, hipStream_t stream);
+                    const float* gate, CombineOut out, hipStream_t stream);
 // The same over weighted bf16 y rows (the prefill tile path).
-void launch_combine_bf16(const uint16_t* y, const int32_t* inv, int T, int k, int H, int has_shared, uint16_t* out,
+void launch_combine_bf16(const uint16_t* y, const int32_t* inv, int T, int k, int H, int has_shared, CombineOut out,
                          hipStream_t stream);
 // Per-wave fallback for any K % 512 == 0 (w4_gemm.hip); max_slots bounds the hit experts + shared.
 void launch_w4_gemm(int mode, bool fp32_scales, int max_slots, const W4StreamParams& p, hipStream_t stream);
@@ -248,7 +256,7 @@ bool fused_down_layout(VerifyParams* vp, int I);
 // out = bf16(sum over slots of w * (sum of the slot row's partial y rows)) (+ gate * shared row),
 // partial rows as VerifyParams::row_seg lists them, fp32 in slot and partial order.
 void launch_combine_parts(const float* ypart, const int2* row_seg, int rps, const int32_t* inv, int T, int k, int H,
-                          int has_shared, const float* wts, const float* gate, uint16_t* out, hipStream_t stream);
+                          int has_shared, const float* wts, const float* gate, CombineOut out, hipStream_t stream);
 // LDS-tiled kernel for long prefill (w4_tile.hip): 96-row passes, column tiles of 512
 // (p.strips = I / 256 for gate_up, H / 512 for down), K % 512 == 0; its gate_up writes one
 // -136*sum(h) per 128 columns and its down reads them that way; its down writes weighted

@@ -789,21 +789,49 @@ __global__ __launch_bounds__(512) void table_prep_kernel(TableParams p) {
   }
 }
 
-// ---------------------------------------------------------------------------
-// Combine: out[t] = sum_slot y[inv[t*k+slot]] (+ y[T*k + t] for the shared
-// expert), fp32 in slot order, one bf16 rounding.  y rows are fp32, or bf16
-// (the prefill tile path, already weighted).  When wts is given the rows
-// are unweighted expert outputs and each is scaled first: by wts[t*k+slot]
-// (the routing weight) or gate[t] (the shared-expert sigmoid) -- the same fp32
-// product the expert epilogues otherwise apply.  grid = (T, H / 512),
-// block = 64: a lane owns 8 columns; the rows are read kBatch at a time, all
-// loads of a batch in flight together, and added in slot order.  fp32 rows come
-// from verify blocks (top-k + the shared expert: 9 rows at top-8), read in one
-// batch of 16; the prefill's bf16 rows stream in batches of 8.
-template <typename YT>
+// Four columns of the layer's output: bf16, or that bf16 value added to the residual in fp32.
+__device__ __forceinline__ void store_combined(const CombineOut& out, int64_t at, float4 v) {
+  const uint32_t lo = f32_to_bf16(v.x) | (static_cast<uint32_t>(f32_to_bf16(v.y)) << 16);
+  const uint32_t hi = f32_to_bf16(v.z) | (static_cast<uint32_t>(f32_to_bf16(v.w)) << 16);
+  if (out.sum == nullptr) {
+    *reinterpret_cast<uint2*>(out.bf16 + at) = make_uint2(lo, hi);
+    return;
+  }
+  float4 r = *reinterpret_cast<const float4*>(out.residual + at);
+  r.x += __uint_as_float(lo << 16);
+  r.y += __uint_as_float(lo & 0xFFFF0000u);
+  r.z += __uint_as_float(hi << 16);
+  r.w += __uint_as_float(hi & 0xFFFF0000u);
+  *reinterpret_cast<float4*>(out.sum + at) = r;
+}
+
+// N columns of the layer's output from `at`: bf16, or (kSum) those bf16 values added to the residual in fp32.
+template <bool kSum, int N>
+__device__ __forceinline__ void store_combined(const CombineOut& out, int64_t at, const float (&v)[N]) {
+  uint32_t pair[N / 2];
+#pragma unroll
+  for (int i = 0; i < N / 2; ++i)
+    pair[i] = f32_to_bf16(v[2 * i]) | (static_cast<uint32_t>(f32_to_bf16(v[2 * i + 1])) << 16);
+  if constexpr (!kSum) {
+    if constexpr (N == 8) *reinterpret_cast<uint4*>(out.bf16 + at) = make_uint4(pair[0], pair[1], pair[2], pair[3]);
+    else *reinterpret_cast<uint2*>(out.bf16 + at) = make_uint2(pair[0], pair[1]);
+  } else {
+#pragma unroll
+    for (int i = 0; i < N / 4; ++i) {
+      float4 r = *reinterpret_cast<const float4*>(out.residual + at + 4 * i);
+      r.x += __uint_as_float(pair[2 * i] << 16);
+      r.y += __uint_as_float(pair[2 * i] & 0xFFFF0000u);
+      r.z += __uint_as_float(pair[2 * i + 1] << 16);
+      r.w += __uint_as_float(pair[2 * i + 1] & 0xFFFF0000u);
+      *reinterpret_cast<float4*>(out.sum + at + 4 * i) = r;
+    }
+  }
+}
+
+template <typename YT, bool kSum>
 __global__ __launch_bounds__(64) void combine_kernel(const YT* __restrict__ y, const int32_t* __restrict__ inv, int T,
                                                      int k, int H, int has_shared, const float* __restrict__ wts,
-                                                     const float* __restrict__ gate, uint16_t* __restrict__ out) {
+                                                     const float* __restrict__ gate, CombineOut out) {
   const int t = blockIdx.x;
   const int c = (blockIdx.y * 64 + threadIdx.x) * 8;
   const int nrows = k + (has_shared ? 1 : 0);
@@ -842,12 +870,7 @@ __global__ __launch_bounds__(64) void combine_kernel(const YT* __restrict__ y, c
         }
       }
     }
-    uint4 o;
-    o.x = f32_to_bf16(acc[0]) | (static_cast<uint32_t>(f32_to_bf16(acc[1])) << 16);
-    o.y = f32_to_bf16(acc[2]) | (static_cast<uint32_t>(f32_to_bf16(acc[3])) << 16);
-    o.z = f32_to_bf16(acc[4]) | (static_cast<uint32_t>(f32_to_bf16(acc[5])) << 16);
-    o.w = f32_to_bf16(acc[6]) | (static_cast<uint32_t>(f32_to_bf16(acc[7])) << 16);
-    *reinterpret_cast<uint4*>(out + static_cast<int64_t>(t) * H + c) = o;
+    store_combined<kSum>(out, static_cast<int64_t>(t) * H + c, acc);
   }
 }
 
@@ -860,7 +883,7 @@ __global__ __launch_bounds__(64) void combine_kernel(const YT* __restrict__ y, c
 __global__ __launch_bounds__(512) void combine_parts_kernel(const float* __restrict__ y, const int2* __restrict__ seg,
                                                             int rps, const int32_t* __restrict__ inv, int T, int k,
                                                             int H, int has_shared, const float* __restrict__ wts,
-                                                            const float* __restrict__ gate, uint16_t* __restrict__ out) {
+                                                            const float* __restrict__ gate, CombineOut out) {
   __shared__ float4 wave_sum[8][64];
   const int t = blockIdx.x, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int c = blockIdx.y * 256 + lane * 4;
@@ -897,10 +920,9 @@ __global__ __launch_bounds__(512) void combine_parts_kernel(const float* __restr
       const float4 u = wave_sum[i][lane];
       o.x += u.x; o.y += u.y; o.z += u.z; o.w += u.w;
     }
-    uint2 r;
-    r.x = f32_to_bf16(o.x) | (static_cast<uint32_t>(f32_to_bf16(o.y)) << 16);
-    r.y = f32_to_bf16(o.z) | (static_cast<uint32_t>(f32_to_bf16(o.w)) << 16);
-    *reinterpret_cast<uint2*>(out + static_cast<int64_t>(t) * H + c) = r;
+    const float v[4] = {o.x, o.y, o.z, o.w};
+    if (out.sum) store_combined<true>(out, static_cast<int64_t>(t) * H + c, v);
+    else store_combined<false>(out, static_cast<int64_t>(t) * H + c, v);
   }
 }
 
@@ -964,21 +986,27 @@ void launch_table_prep(const TableParams& p, hipStream_t stream) {
 }
 
 void launch_combine(const float* y, const int32_t* inv, int T, int k, int H, int has_shared, const float* wts,
-                    const float* gate, uint16_t* out, hipStream_t stream) {
+                    const float* gate, CombineOut out, hipStream_t stream) {
   if (T <= 0) return;
-  hipLaunchKernelGGL(combine_kernel<float>, dim3(T, (H + 511) / 512), dim3(64), 0, stream, y, inv, T, k, H, has_shared,
-                     wts, gate, out);
+  const dim3 grid(T, (H + 511) / 512), block(64);
+  if (out.sum)
+    hipLaunchKernelGGL((combine_kernel<float, true>), grid, block, 0, stream, y, inv, T, k, H, has_shared, wts, gate, out);
+  else
+    hipLaunchKernelGGL((combine_kernel<float, false>), grid, block, 0, stream, y, inv, T, k, H, has_shared, wts, gate, out);
 }
 
-void launch_combine_bf16(const uint16_t* y, const int32_t* inv, int T, int k, int H, int has_shared, uint16_t* out,
+void launch_combine_bf16(const uint16_t* y, const int32_t* inv, int T, int k, int H, int has_shared, CombineOut out,
                          hipStream_t stream) {
   if (T <= 0) return;
-  hipLaunchKernelGGL(combine_kernel<uint16_t>, dim3(T, (H + 511) / 512), dim3(64), 0, stream, y, inv, T, k, H,
-                     has_shared, nullptr, nullptr, out);
+  const dim3 grid(T, (H + 511) / 512), block(64);
+  if (out.sum)
+    hipLaunchKernelGGL((combine_kernel<uint16_t, true>), grid, block, 0, stream, y, inv, T, k, H, has_shared, nullptr, nullptr, out);
+  else
+    hipLaunchKernelGGL((combine_kernel<uint16_t, false>), grid, block, 0, stream, y, inv, T, k, H, has_shared, nullptr, nullptr, out);
 }
 
 void launch_combine_parts(const float* ypart, const int2* row_seg, int rps, const int32_t* inv, int T, int k, int H,
-                          int has_shared, const float* wts, const float* gate, uint16_t* out, hipStream_t stream) {
+                          int has_shared, const float* wts, const float* gate, CombineOut out, hipStream_t stream) {
   if (T <= 0) return;
   hipLaunchKernelGGL(combine_parts_kernel, dim3(T, (H + 255) / 256), dim3(512), 0, stream, ypart, row_seg, rps, inv, T,
                      k, H, has_shared, wts, gate, out);

@@ -438,6 +438,33 @@ def moe_w4a16(hidden: torch.Tensor, gate_up: PackedW4, down: PackedW4, *, top_k:
     return out
 
 
+def moe_w4a16_add(residual: torch.Tensor, hidden: torch.Tensor, gate_up: PackedW4, down: PackedW4, *, top_k: int,
+                  router_weight: torch.Tensor, shared: Optional[SharedExpert] = None,
+                  workspace: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """``residual + moe_w4a16(hidden, ...)`` in fp32 ``[T, H]`` without a launch for the add; ``residual`` is contiguous
+    fp32 of hidden's shape."""
+    device, flat, sgu, sdn, sgate = _moe_common(hidden, gate_up, down, shared)
+    t, h = flat.shape
+    e = gate_up.experts
+    if not _as(residual, torch.float32, (t, h), device):
+        raise ValueError(f"residual must be a contiguous float32 [{t}, {h}] tensor on {device}")
+    _require_device(router_weight)
+    if router_weight.dtype != torch.bfloat16 or tuple(router_weight.shape) != (e, h):
+        raise ValueError(f"router_weight must be bfloat16 [{e}, {h}]")
+    rw = router_weight.contiguous()
+    logits = torch.empty((t, e), dtype=torch.float32, device=device)
+    r = _routing_buffers(t, e, top_k, device)
+    out = torch.empty_like(residual)
+    ws = _workspace(_lib.load().dflash_moe_workspace_bytes(t, h, gate_up.rows // 2, e, top_k, gate_up.group_size,
+                                                           int(shared is not None)), device, workspace)
+    gu, dn = _desc(gate_up), _desc(down)
+    _lib.call("dflash_moe_w4a16_residual", _ptr(flat), t, h, _ptr(rw), top_k, ctypes.byref(gu), ctypes.byref(dn),
+              None if sgu is None else ctypes.byref(sgu), None if sdn is None else ctypes.byref(sdn), _ptr(sgate),
+              _ptr(residual), _ptr(out), _ptr(logits), _ptr(r.ids), _ptr(r.weights), _ptr(r.perm), _ptr(r.inv),
+              _ptr(r.offsets), _ptr(ws), ws.numel(), _stream(device))
+    return out
+
+
 NOALLOC_SCRATCH_BYTES = 8 << 20
 
 

@@ -349,7 +349,8 @@ class TargetModel:
             pending = rest[0] if rest else None
             if trace is not None:
                 trace.update(mid=mid, moe_in=normed)
-            return mid + self._moe(normed, lw, workspace), pending         # bf16 joins the fp32 sum exactly
+            return ops.moe_w4a16_add(mid, normed, lw.gate_up, lw.down, top_k=c.top_k, router_weight=lw.router,
+                                     shared=lw.shared, workspace=workspace), pending
         normed = layers.rms_normalise(hidden, lw.input_norm, c.rms_eps, 1.0).to(torch.bfloat16)
         if lw.kind == "linear_attention":
             mixed, pending = self._gdn(normed, lw, state.conv[i], state.recurrent[i])

@@ -91,3 +91,26 @@ def test_attention_layer_matches_oracle(pkg, device, tokens, context, heads, kv_
     assert metrics.compare(state.values[0][0, :, rows].float().cpu(), ref["values"])["max_rel"] <= TOL
     assert torch.equal(state.keys[0][:, :, context + tokens:], untouched)
     assert torch.equal(state.keys[0][0, :, :context].cpu(), before["keys"][:, :context])
+
+
+def test_attention_layer_over_more_splits_than_lanes(pkg, device):
+    """66 splits of the keys: the merge takes two of them in some lanes."""
+    test_attention_layer_matches_oracle(pkg, device, 1, 8400, 16, 2, 256)
+
+
+@pytest.mark.parametrize("tokens,split_down", [(1, False), (16, False), (16, True), (40, False), (260, False)])
+def test_moe_with_the_residual_add(pkg, device, tokens, split_down):
+    """The layer that leaves residual + output equals the layer and the add bit for bit, on every path with a combine of
+    its own (verify block, its split down, the work-table kernels, the prefill tiles)."""
+    layer = pkg.synthetic.moe_layer(tokens, hidden=512, inter=512, experts=16, seed=tokens)
+    shared = pkg.SharedExpert(layer.shared.gate_up.to(device), layer.shared.down.to(device),
+                              layer.shared.gate_weight.to(device))
+    args = dict(top_k=4, router_weight=layer.router_weight.to(device), shared=shared)
+    x, banks = layer.hidden.to(device), (layer.gate_up.to(device), layer.down.to(device))
+    residual = torch.randn((tokens, 512), generator=torch.Generator().manual_seed(1)).to(device)
+    with pkg.ops.split_down(split_down):
+        want = residual + pkg.ops.moe_w4a16(x, *banks, **args)
+        got = pkg.ops.moe_w4a16_add(residual, x, *banks, **args)
+    assert torch.equal(got, want)
+    with pytest.raises(ValueError, match="residual"):
+        pkg.ops.moe_w4a16_add(residual.to(torch.bfloat16), x, *banks, **args)
