@@ -7,10 +7,13 @@ is raised with the library's own message.
 from __future__ import annotations
 
 import ctypes
+import importlib.machinery
+import importlib.util
 from pathlib import Path
 
 PACKAGE_DIR = Path(__file__).resolve().parent
 LIBRARY_PATH = PACKAGE_DIR / "libdflash_hip.so"
+HOST_PATH = PACKAGE_DIR / "dflash_host.so"
 
 ABI_VERSION = 6
 DTYPE_BF16 = 0
@@ -165,6 +168,25 @@ def load(path: Path = LIBRARY_PATH) -> ctypes.CDLL:
         raise RuntimeError(f"libdflash_hip.so ABI {version} != expected {ABI_VERSION}")
     _LIB = lib
     return lib
+
+
+_HOST = None
+
+
+def host():
+    """The native form of ops.py's plain calls (``csrc/host.cpp``), bound (once) to the loaded library's entries."""
+    global _HOST
+    if _HOST is None:
+        from .packing import PackedW4, SharedExpert
+        lib = load()
+        if not HOST_PATH.is_file():
+            raise RuntimeError(f"{HOST_PATH.name} not found at {HOST_PATH}; build it with build.py")
+        loader = importlib.machinery.ExtensionFileLoader("dflash_host", str(HOST_PATH))
+        module = importlib.util.module_from_spec(importlib.util.spec_from_loader("dflash_host", loader))
+        loader.exec_module(module)
+        module.bind(PackedW4, SharedExpert, lambda name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value)
+        _HOST = module
+    return _HOST
 
 
 def check(function: str, status: int) -> None:

@@ -1,4 +1,5 @@
-"""Build recipe for ``libdflash_hip.so`` (hand-written HIP for gfx950 only).
+"""Build recipe for ``libdflash_hip.so`` (hand-written HIP for gfx950 only) and ``dflash_host.so`` (the native form
+of ops.py's plain calls: C++ over torch's headers, no device code).
 
 ``python build.py`` from this directory, or ``build()`` from Python.  Each
 translation unit is compiled in parallel with hipcc, then linked into one
@@ -13,6 +14,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 import tempfile
 from pathlib import Path
 
@@ -22,6 +24,8 @@ TIMELINE_LIBRARY = PACKAGE_DIR / "libdflash_hip_timeline.so"
 SOURCES = ("csrc/api.hip", "csrc/route.hip", "csrc/w4_gemm.hip", "csrc/w4_stream.hip",
            "csrc/w4_tile.hip", "csrc/w4_verify.hip", "csrc/w4_small.hip", "csrc/w4_linear.hip",
            "csrc/repack.hip", "csrc/gdn.hip", "csrc/attention.hip")
+HOST_SOURCE = "csrc/host.cpp"
+HOST_LIBRARY = PACKAGE_DIR / "dflash_host.so"
 ARCH = "gfx950"
 FLAGS = (
     f"--offload-arch={ARCH}", "-O3", "-std=c++17", "-fPIC",
@@ -37,6 +41,17 @@ def _hipcc() -> str:
     return path
 
 
+def _host_command(output: Path) -> list:
+    import torch
+    root = Path(torch.__file__).resolve().parent
+    include = (root / "include", root / "include/torch/csrc/api/include", sysconfig.get_paths()["include"],
+               "/opt/rocm/include")
+    return [shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden",
+            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-DUSE_ROCM=1", "-D__HIP_PLATFORM_AMD__=1",
+            *(f"-I{i}" for i in include), str(PACKAGE_DIR / HOST_SOURCE), "-o", str(output), f"-L{root / 'lib'}",
+            "-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip"]
+
+
 def build(verbose: bool = False, timeline: bool = False) -> Path:
     hipcc = _hipcc()
     target = TIMELINE_LIBRARY if timeline else LIBRARY
@@ -48,10 +63,14 @@ def build(verbose: bool = False, timeline: bool = False) -> Path:
             cmd = [hipcc, *flags, "-c", str(PACKAGE_DIR / src), "-o", str(obj)]
             objects.append(obj)
             procs.append((cmd, subprocess.Popen(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)))
+        host = None if timeline else Path(tmp) / HOST_LIBRARY.name
+        if host:
+            cmd = _host_command(host)
+            procs.append((cmd, subprocess.Popen(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)))
         for cmd, proc in procs:
             out, _ = proc.communicate()
             if proc.returncode:
-                raise RuntimeError(f"hipcc failed ({proc.returncode}): {' '.join(cmd)}\n{out}")
+                raise RuntimeError(f"compiler failed ({proc.returncode}): {' '.join(cmd)}\n{out}")
             if verbose and out.strip():
                 print(out)
         staged = Path(tmp) / target.name
@@ -59,9 +78,11 @@ def build(verbose: bool = False, timeline: bool = False) -> Path:
         proc = subprocess.run(link, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
         if proc.returncode:
             raise RuntimeError(f"link failed: {' '.join(link)}\n{proc.stdout}")
-        tmp_target = target.with_suffix(".so.tmp")
-        shutil.copyfile(staged, tmp_target)
-        os.replace(tmp_target, target)
+        for built, final in ((staged, target), (host, HOST_LIBRARY)):
+            if built:
+                tmp_target = final.with_suffix(".so.tmp")
+                shutil.copyfile(built, tmp_target)
+                os.replace(tmp_target, final)
     return target
 
 

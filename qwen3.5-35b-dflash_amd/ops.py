@@ -120,10 +120,19 @@ def to_tiled(w: PackedW4) -> PackedW4:
     return PackedW4(packed, scales, w.group_size, "tiled")
 
 
+def _plain(x) -> bool:
+    """Whether a call on ``x`` is first offered to the native form (``csrc/host.cpp``), which takes it or returns None."""
+    return type(x) is torch.Tensor and x.is_cuda
+
+
 def qlinear(x: torch.Tensor, weight: PackedW4, *, workspace: Optional[torch.Tensor] = None,
             out_dtype: torch.dtype = torch.bfloat16) -> torch.Tensor:
     """W4A16 linear ``x[..., K] -> [..., N]`` (bf16 in, fp32 accumulation; bf16 out, or the
     unrounded fp32 sums with ``out_dtype=torch.float32``)."""
+    if workspace is None and _plain(x) and (out_dtype is torch.bfloat16 or out_dtype is torch.float32):
+        y = _lib.host().linear(x, weight, out_dtype is torch.float32)
+        if y is not None:
+            return y
     weight.validate("weight")
     if weight.packed.ndim != 2:
         raise ValueError("qlinear takes one packed matrix [N, K/2]")
@@ -179,6 +188,23 @@ def gdn_mixer(hidden: torch.Tensor, history: torch.Tensor, state: torch.Tensor, 
     return r
 
 
+def gdn_mixer_plain(hidden, history, state, *, in_proj, out_proj, input_norm, post_norm, norm, a_log, dt_bias, conv,
+                    key_heads, eps) -> Optional[GdnMixer]:
+    """:func:`gdn_mixer` of arguments :func:`gdn_mixer_fits` accepts, both in one native call; None for others."""
+    r = _plain(hidden) and _lib.host().gdn(hidden, history, state, in_proj, out_proj, input_norm, post_norm, norm, a_log,
+                                           dt_bias, conv, key_heads, eps)
+    return GdnMixer(*r) if r else None
+
+
+def attention_mixer_plain(hidden, keys, values, position, *, in_proj, out_proj, input_norm, post_norm, q_norm, k_norm,
+                          inv_freq, heads, kv_heads, head_dim, eps) -> Optional[tuple]:
+    """:func:`attention_mixer` of arguments :func:`attention_mixer_fits` accepts, both in one native call; None for
+    others."""
+    r = _plain(hidden) and _lib.host().attention(hidden, keys, values, position, in_proj, out_proj, input_norm, post_norm,
+                                                 q_norm, k_norm, inv_freq, heads, kv_heads, head_dim, eps)
+    return r or None
+
+
 def _as(t, dtype: torch.dtype, shape: tuple, device: torch.device) -> bool:
     """Whether ``t`` is what a kernel reads as is: this dtype, shape and device, contiguous, 16-byte aligned."""
     return (isinstance(t, torch.Tensor) and t.dtype == dtype and t.shape == shape and t.device == device
@@ -224,6 +250,10 @@ def gdn_commit(state: torch.Tensor, keys: torch.Tensor, u: torch.Tensor, cum: to
     """``(recurrent state, conv history)`` after the first ``accepted`` tokens of one chunk of :func:`gdn_mixer`
     (``layers.state_after`` and the window's columns ``[first, first + 3)``) in one launch; ``None`` when the tensors
     are not laid out as that call leaves them."""
+    if _plain(state):
+        done = _lib.host().commit(state, keys, u, cum, accepted, window, first)
+        if done is not None:
+            return done
     hv, device = state.shape[1], state.device
     if (device.type != "cuda" or not 1 <= accepted <= 16 or not _as(state, torch.float32, (1, hv, 128, 128), device)
             or keys.shape[:2] != (1, hv) or keys.shape[2] < accepted or keys.shape[3] != 128 or u.shape != keys.shape
@@ -403,6 +433,10 @@ def moe_w4a16(hidden: torch.Tensor, gate_up: PackedW4, down: PackedW4, *, top_k:
     With ``return_routing=True`` also returns ``(Routing, logits)``; ``logits``
     are the fp32 router logits the routing was computed from.
     """
+    if router_logits is None and not return_routing and _plain(hidden):
+        out = _lib.host().moe(hidden, gate_up, down, top_k, router_weight, shared, workspace, None)
+        if out is not None:
+            return out
     device, flat, sgu, sdn, sgate = _moe_common(hidden, gate_up, down, shared)
     if type(top_k) is not int:
         raise ValueError("top_k must be an int")
@@ -443,6 +477,10 @@ def moe_w4a16_add(residual: torch.Tensor, hidden: torch.Tensor, gate_up: PackedW
                   workspace: Optional[torch.Tensor] = None) -> torch.Tensor:
     """``residual + moe_w4a16(hidden, ...)`` in fp32 ``[T, H]`` without a launch for the add; ``residual`` is contiguous
     fp32 of hidden's shape."""
+    if _plain(hidden):
+        out = _lib.host().moe(hidden, gate_up, down, top_k, router_weight, shared, workspace, residual)
+        if out is not None:
+            return out
     device, flat, sgu, sdn, sgate = _moe_common(hidden, gate_up, down, shared)
     t, h = flat.shape
     e = gate_up.experts

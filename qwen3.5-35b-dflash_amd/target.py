@@ -315,10 +315,14 @@ class TargetModel:
         c, args = self.config, self._gdn_args(lw)
         if c.linear_key_dim != 128 or c.linear_value_dim != 128 or c.linear_value_heads != lw.a_log.shape[0]:
             return None
-        if not ops.gdn_mixer_fits(hidden, conv_hist, state, **args):
-            return None
-        r = ops.gdn_mixer(hidden, conv_hist, state, **args)
+        r = ops.gdn_mixer_plain(hidden, conv_hist, state, **args)
+        if r is None:
+            if not ops.gdn_mixer_fits(hidden, conv_hist, state, **args):
+                return None
+            r = ops.gdn_mixer(hidden, conv_hist, state, **args)
         n = layers.CHUNK
+        if hidden.shape[0] <= n:
+            return r.mid, r.normed, GdnPending(r.window, state, [layers.DeltaChunk(r.core, r.states[0], r.keys, r.u, r.cum)])
         chunks = [layers.DeltaChunk(*f) for f in zip(r.core.split(n, 2), r.states.unbind(0), r.keys.split(n, 2),
                                                      r.u.split(n, 2), r.cum.split(n, 2))]
         return r.mid, r.normed, GdnPending(r.window, state, chunks)
@@ -330,6 +334,9 @@ class TargetModel:
         args = dict(in_proj=lw.mixer_in, out_proj=lw.mixer_out, input_norm=lw.input_norm, post_norm=lw.post_norm,
                     q_norm=lw.q_norm, k_norm=lw.k_norm, inv_freq=self.inv_freq, heads=c.heads, kv_heads=c.kv_heads,
                     head_dim=c.head_dim, eps=c.rms_eps)
+        done = ops.attention_mixer_plain(hidden, keys, values, pos, **args)
+        if done is not None:
+            return done
         if not ops.attention_mixer_fits(hidden, keys, values, pos, **args):
             return None
         return ops.attention_mixer(hidden, keys, values, pos, **args)

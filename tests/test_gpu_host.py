@@ -1,0 +1,114 @@
+"""GPU: the native form of ops.py's plain calls (``csrc/host.cpp``) against the Python form of the same calls.
+
+Both enqueue the same kernels with the same arguments, so results are equal bit for bit; what the native form does not
+take (views, other types, subclasses, modes) it leaves to the Python form, errors included.
+"""
+import pytest
+import torch
+from torch.utils._python_dispatch import TorchDispatchMode
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture
+def python_form(pkg, monkeypatch):
+    """Calls a function with the native form switched off."""
+    def call(fn, *args, **kw):
+        with monkeypatch.context() as m:
+            m.setattr(pkg.ops, "_plain", lambda x: False)
+            return fn(*args, **kw)
+    return call
+
+
+def _weight(pkg, device, n, k, group=128, dtype=torch.bfloat16, layout="tiled", seed=0):
+    w = pkg.synthetic.int4_weight(torch.Generator().manual_seed(seed), (n, k), group, dtype).to(device)
+    return w.tiled() if layout == "tiled" else w
+
+
+@pytest.mark.parametrize("shape", [(2048,), (1, 2048), (2, 3, 2048), (70, 2048)])
+@pytest.mark.parametrize("group,dtype,layout", [(128, torch.bfloat16, "tiled"), (256, torch.float32, "portable")])
+def test_linear(pkg, device, python_form, shape, group, dtype, layout):
+    w = _weight(pkg, device, 96, 2048, group, dtype, layout)
+    x = torch.randn(shape, device=device).to(torch.bfloat16)
+    for out_dtype in (torch.bfloat16, torch.float32):
+        y = pkg._lib.host().linear(x, w, out_dtype is torch.float32)
+        want = python_form(pkg.ops.qlinear, x, w, out_dtype=out_dtype)
+        assert y is not None and y.dtype == out_dtype and y.shape == (*shape[:-1], 96) and torch.equal(y, want)
+
+
+def test_linear_leaves_other_forms(pkg, device, python_form):
+    w, x = _weight(pkg, device, 96, 512), torch.randn((8, 512), device=device).to(torch.bfloat16)
+    native = pkg._lib.host().linear
+    strided = torch.randn((8, 1024), device=device).to(torch.bfloat16)[:, ::2]
+    assert native(strided, w, False) is None
+    assert torch.equal(pkg.ops.qlinear(strided, w), pkg.ops.qlinear(strided.contiguous(), w))
+    offset = torch.randn((8 * 512 + 1,), device=device).to(torch.bfloat16)[1:].view(8, 512)      # 2-byte aligned
+    for bad, error in ((offset, pkg._lib.DflashError), (x.float(), ValueError), (x[:, :256], ValueError), (x.cpu(), ValueError)):
+        with pytest.raises(error):
+            pkg.ops.qlinear(bad, w)
+    assert pkg.ops.qlinear(x[:0], w).shape == (0, 96)
+    for bad in (w._replace(group_size=64), w._replace(layout="other"), w._replace(scales=w.scales.half()),
+                w._replace(scales=w.scales[:, :1]), w._replace(packed=w.packed.cpu())):
+        assert native(x, bad, False) is None
+        with pytest.raises(ValueError):
+            pkg.ops.qlinear(x, bad)
+    assert native(x, tuple(w), False) is None
+
+    class Mode(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+    with Mode():
+        assert native(x, w, False) is None
+        assert pkg.ops.qlinear(x, w).shape == (8, 96)
+
+
+@pytest.mark.parametrize("tokens,shared", [(1, True), (16, False), (40, True)])
+def test_moe(pkg, device, python_form, tokens, shared):
+    layer = pkg.synthetic.moe_layer(tokens, hidden=512, inter=512, experts=16, seed=tokens)
+    x, banks = layer.hidden.to(device), (layer.gate_up.to(device), layer.down.to(device))
+    sh = pkg.SharedExpert(layer.shared.gate_up.to(device), layer.shared.down.to(device), layer.shared.gate_weight.to(device))
+    router, native = layer.router_weight.to(device), pkg._lib.host().moe
+    args = dict(top_k=4, router_weight=router, shared=sh if shared else None)
+    want = python_form(pkg.ops.moe_w4a16, x, *banks, **args)
+    need = pkg.ops.moe_workspace_bytes(tokens, 512, 512, 16, 4, 128, shared)
+    for ws in (None, torch.empty(need, dtype=torch.uint8, device=device)):
+        got = native(x, *banks, 4, router, args["shared"], ws, None)
+        assert got is not None and torch.equal(got, want)
+    assert native(x, *banks, 4, router, args["shared"], torch.empty(need - 1, dtype=torch.uint8, device=device), None) is None
+    assert native(x, *banks, 4, router.t().contiguous().t(), args["shared"], None, None) is None
+    for k in (0, 17, True, 4.0):
+        assert native(x, *banks, k, router, args["shared"], None, None) is None
+
+
+@pytest.mark.parametrize("kind", ["linear_attention", "full_attention"])
+@pytest.mark.parametrize("tokens", [1, 16, 30])
+def test_layer(pkg, device, python_form, kind, tokens):
+    c = pkg.target.small_config((kind,))
+    model = pkg.target.TargetModel(pkg.target.random_weights(c, seed=3, device=device, layout="tiled"), capacity=80)
+    x = torch.randn((tokens, c.hidden), device=device)
+
+    def run():
+        state = model.synthetic_context(9, seed=4)
+        hidden, pending = model.layer(0, x, state)
+        model.commit(state, pkg.target.Pending(9, tokens, [pending]), max(1, tokens - 3))
+        return [hidden, *state.conv, *state.recurrent, *state.keys, *state.values]
+    for a, b in zip(run(), python_form(run)):
+        assert (a is None and b is None) or torch.equal(a, b)
+
+
+def test_calls_run_on_the_current_stream(pkg, device):
+    """A call inside a stream context is ordered on that stream: behind work queued there, before what follows."""
+    w, stream = _weight(pkg, device, 512, 2048), torch.cuda.Stream(device)
+    x = torch.randn((16, 2048), device=device).to(torch.bfloat16)
+    want = pkg.ops.qlinear(x, w)
+    torch.cuda.synchronize()
+    late = torch.zeros_like(x)
+    with torch.cuda.stream(stream):
+        big = torch.randn((4096, 4096), device=device)
+        for _ in range(8):
+            big = big @ big
+            big /= big.norm()
+        late.copy_(x)
+        y = pkg.ops.qlinear(late, w)
+    stream.synchronize()
+    assert torch.equal(y, want)
