@@ -18,11 +18,11 @@
 //       size 102 us; the 16-column streaming kernel that served these sizes before 267 us; 105 us among other calls).
 //   w4_linear_split_kernel  for outputs of few tiles: a workgroup takes 32 rows x 64 columns, its four waves every fourth
 //       k-block each, operands straight into MFMA fragment registers, the four partial sums added in LDS in wave order.
-//       Bound by the latency of its loads: 333 x 2048 x 4096 in 28 us with the prep launch (4 us), 495 us on the
+//       Bound by the latency of its loads: 333 x 2048 x 4096 in 24 us with the prep launch (4 us), 495 us on the
 //       per-wave kernel before.
 //
 // The line between them: tile when its tiles fill at least 5/8 of the CUs.  Measured, split / tile, us: 80 tiles 17.7 /
-// 22.9 (300 x 4096 x 2048) and 39.8 / 50.5 (600 x 2048 x 4096); 160 tiles 25.2 / 25.2 (600 x 4096 x 2048); 196
+// 22.9 (300 x 4096 x 2048) and 33.1 / 50.5 (600 x 2048 x 4096, portable); 160 tiles 25.2 / 25.2 (600 x 4096 x 2048); 196
 // tiles 26.1 / 24.1 (200 x 12352 x 2048); 256 tiles 34.1 / 26.7 (1024 x 4096 x 2048).
 //
 // Against 64 bits the fp32 sums are 1.0e-7 (split) and 2.1e-7 to 2.6e-7 (tile) off, relative (1.0e-6 to 2.8e-6
@@ -136,12 +136,17 @@ struct Weights {
     }
   }
   __device__ __forceinline__ void load(int kb, uint4 (&w)[2][2], uint32_t (&s)[2]) const {
-    const int so = __builtin_amdgcn_readfirstlane(static_cast<int>((kb >> gshift) * sg));
     const int wo = __builtin_amdgcn_readfirstlane(static_cast<int>(kb * wkb));
 #pragma unroll
-    for (int f = 0; f < 2; ++f) {
+    for (int f = 0; f < 2; ++f)
 #pragma unroll
       for (int q = 0; q < 2; ++q) w[f][q] = buf_load16(wrs, woff[f], wo + q * jj);
+    load_scales(kb, s);
+  }
+  __device__ __forceinline__ void load_scales(int kb, uint32_t (&s)[2]) const {
+    const int so = __builtin_amdgcn_readfirstlane(static_cast<int>((kb >> gshift) * sg));
+#pragma unroll
+    for (int f = 0; f < 2; ++f) {
       s[f] = sizeof(ScaleT) == 4 ? __builtin_amdgcn_raw_buffer_load_b32(srs, static_cast<int>(soff[f]), so, 0)
                                  : static_cast<uint32_t>(__builtin_amdgcn_raw_buffer_load_b16(srs, static_cast<int>(soff[f]), so, 0));
     }
@@ -152,6 +157,10 @@ struct Weights {
 constexpr int kSub = 2;  // 32-row subtiles of a tile
 
 typedef __attribute__((address_space(3))) void* lds_ptr;
+// 16 bytes a lane straight into LDS (lane l at dst + 16 l)
+__device__ __forceinline__ void dma16(buf_rsrc r, void* dst, uint32_t voff, uint32_t soff) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_ptr)dst, 16, static_cast<int>(voff), static_cast<int>(soff), 0, 0);
+}
 
 template <int N>
 struct Int {
@@ -200,8 +209,8 @@ __global__ __launch_bounds__(256, 3) void w4_linear_tile_kernel(LinearParams p) 
     for (int ms = 0; ms < kSub; ++ms)
 #pragma unroll
       for (int q = 0; q < 2; ++q)  // wave w: fragments w and w + 4 of every subtile
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(ars, (lds_ptr)((S ? a1 : a0) + (ms * 8 + q * 4 + wave) * 64), 16, lane * 16,
-                                                 (min(ms, live - 1) * nkb + kb) * 8192 + (q * 4 + wave) * 1024, 0, 0);
+        dma16(ars, (S ? a1 : a0) + (ms * 8 + q * 4 + wave) * 64, lane * 16,
+              (min(ms, live - 1) * nkb + kb) * 8192 + (q * 4 + wave) * 1024);
     __builtin_amdgcn_raw_ptr_buffer_load_lds(nrs, (lds_ptr)((S ? n1 : n0) + wave * 64), 4, static_cast<int>(noff), kb * 128, 0, 0);
     weights.load(kb, wb[S], sb[S]);
     asm volatile("" ::: "memory");
@@ -333,9 +342,12 @@ __global__ __launch_bounds__(256, 3) void w4_linear_tile_kernel(LinearParams p) 
 }
 
 // ------------------------------------------------------------------ k split over the waves
-template <typename ScaleT>
+// kStaged (portable banks): a wave's weights of a k-block reach LDS by four direct-to-LDS loads of 16 whole 64-byte row
+// pieces each, and lanes read their fragments from there; straight into registers each load would take 32 bytes of 32
+// rows (333 x 2048 x 4096 28.7 -> 24.1 us, 600 x 2048 x 4096 39.3 -> 33.1).  Tiled banks lie in fragment order already.
+template <typename ScaleT, bool kStaged>
 __global__ __launch_bounds__(256, 2) void w4_linear_split_kernel(LinearParams p) {
-  __shared__ f32x4 part[4][8][64];
+  __shared__ f32x4 part[4][8][64];  // a wave's eight kilobytes are also its two weight stages, [64 rows][4 pieces] each
   const int N = p.N, nkb = p.K >> 7;
   const int mt_count = (p.M + 31) >> 5, nt_count = (N + 63) >> 6;
   int mt, nt;
@@ -353,9 +365,35 @@ __global__ __launch_bounds__(256, 2) void w4_linear_split_kernel(LinearParams p)
     uint32_t s[2];
     f32x4 neg[4];
   };
-  auto load = [&](int kb, Block& b) {
+  // staged: load i takes rows 16 i .. 16 i + 15, lane l piece (l & 3) ^ (row / 2 & 3) of row 16 i + l / 4, so that the
+  // lanes that read one piece of consecutive rows do not meet in a bank
+  uint4* const own[2] = {reinterpret_cast<uint4*>(part[wave]), reinterpret_cast<uint4*>(part[wave] + 4)};
+  uint32_t goff[4], loff[2][2];
+  if constexpr (kStaged) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int row = 16 * i + (lane >> 2);  // columns past N repeat the last fragment's
+      goff[i] = static_cast<uint32_t>(min(row, cols - 32 + (row & 31))) * (static_cast<uint32_t>(p.K) >> 1) +
+                ((lane & 3) ^ (row >> 1 & 3)) * 16u;
+    }
+#pragma unroll
+    for (int f = 0; f < 2; ++f)
+#pragma unroll
+      for (int q = 0; q < 2; ++q) loff[f][q] = (f * 32 + r) * 4 + ((2 * q + h) ^ (r >> 1 & 3));
+  }
+  auto load = [&](int kb, Block& b, uint4* stage) {
     kb = __builtin_amdgcn_readfirstlane(kb);
-    weights.load(kb, b.w, b.s);
+    if constexpr (kStaged) {
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the block that lay there has been read
+      asm volatile("" ::: "memory");
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        dma16(weights.wrs, stage + i * 64, goff[i], kb * 64);
+      weights.load_scales(kb, b.s);
+    } else {
+      weights.load(kb, b.w, b.s);
+    }
 #pragma unroll
     for (int j = 0; j < 8; ++j) b.x[j] = buf_load16(xrs, lane * 16, kb * 8192 + j * 1024);
 #pragma unroll
@@ -364,7 +402,18 @@ __global__ __launch_bounds__(256, 2) void w4_linear_split_kernel(LinearParams p)
     __builtin_amdgcn_sched_barrier(0);  // issued here, a k-block ahead of their use
   };
   f32x16 tot[2] = {zero16(), zero16()};
-  auto compute = [&](const Block& b) {
+  auto compute = [&](Block& b, const uint4* stage) {
+    if constexpr (kStaged) {
+      // this block's loads are in once only the next one's (4 + 2 + 8 + 4) are pending; written out, since the compiler's
+      // own wait for direct-to-LDS loads can be missing in a loop
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_s_waitcnt(0x0F70 | (18 & 15) | (18 >> 4) << 14);  // vmcnt(18)
+      asm volatile("" ::: "memory");
+#pragma unroll
+      for (int f = 0; f < 2; ++f)
+#pragma unroll
+        for (int q = 0; q < 2; ++q) b.w[f][q] = stage[loff[f][q]];
+    }
 #pragma unroll
     for (int f = 0; f < 2; ++f) {
       f32x16 acc;
@@ -378,15 +427,16 @@ __global__ __launch_bounds__(256, 2) void w4_linear_split_kernel(LinearParams p)
   // wave w: k-blocks w, w + 4, ... (the four waves read neighbouring blocks of a weight row, whole cache lines of it in
   // the portable layout, at about the same time)
   Block b0, b1;
-  load(min(wave, nkb - 1), b0);  // past the last k-block it is loaded again: a load under a condition would make every use wait for all
+  load(min(wave, nkb - 1), b0, own[0]);  // past the last k-block it is loaded again: a load under a condition would make every use wait for all
 #pragma unroll 1
   for (int kb = wave; kb < nkb; kb += 8) {
-    load(min(kb + 4, nkb - 1), b1);
-    compute(b0);
+    load(min(kb + 4, nkb - 1), b1, own[1]);
+    compute(b0, own[0]);
     if (kb + 4 >= nkb) break;
-    load(min(kb + 8, nkb - 1), b0);
-    compute(b1);
+    load(min(kb + 8, nkb - 1), b0, own[0]);
+    compute(b1, own[1]);
   }
+  if constexpr (kStaged) __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): part holds no stage any more
 #pragma unroll
   for (int f = 0; f < 2; ++f)
 #pragma unroll
@@ -434,8 +484,13 @@ void launch_w4_linear(const LinearParams& p, int cus, hipStream_t stream) {
   } else {
     const int64_t parts = static_cast<int64_t>((p.M + 31) / 32) * ((p.N + 63) / 64);
     const dim3 grid(static_cast<unsigned>((parts + 7) / 8 * 8)), block(256);
-    if (p.scale_f32) hipLaunchKernelGGL(w4_linear_split_kernel<float>, grid, block, 0, stream, p);
-    else hipLaunchKernelGGL(w4_linear_split_kernel<uint16_t>, grid, block, 0, stream, p);
+    if (p.tiled) {
+      if (p.scale_f32) hipLaunchKernelGGL((w4_linear_split_kernel<float, false>), grid, block, 0, stream, p);
+      else hipLaunchKernelGGL((w4_linear_split_kernel<uint16_t, false>), grid, block, 0, stream, p);
+    } else {
+      if (p.scale_f32) hipLaunchKernelGGL((w4_linear_split_kernel<float, true>), grid, block, 0, stream, p);
+      else hipLaunchKernelGGL((w4_linear_split_kernel<uint16_t, true>), grid, block, 0, stream, p);
+    }
   }
 }
 
