@@ -253,6 +253,7 @@ int dflash_moe_w4a16_noalloc(const void* hidden, int64_t tokens, int64_t hidden_
  * [hidden_size][128 * value_heads].  Norm weights are applied as w + 1 (input_norm, post_norm) and w (norm).
  * Outputs besides mid fp32 [T][hidden_size] and normed bf16: what commits any prefix of the block needs --
  * window bf16 [C][3 + T] (conv history, then the block's columns; C = 128 * (2 * key_heads + value_heads)),
+ * tail bf16 [C][3] (its last columns: the conv history after the whole block),
  * keys, u, core fp32 [value_heads][T][128], cum fp32 [value_heads][T] (log decay summed inside each chunk of 16
  * tokens) and states fp32 [ceil(T / 16)][value_heads][128][128] (the state after each chunk).
  */
@@ -269,8 +270,12 @@ typedef struct dflash_gdn {
 } dflash_gdn;
 size_t dflash_gdn_workspace_bytes(int64_t tokens, int64_t hidden_size, int64_t key_heads, int64_t value_heads);
 int dflash_gdn_mixer(const dflash_gdn* g, const float* hidden, int64_t tokens, const void* history, const float* state,
-                     float* mid, void* normed, void* window, float* states, float* keys, float* u, float* cum,
+                     float* mid, void* normed, void* window, void* tail, float* states, float* keys, float* u, float* cum,
                      float* core, void* workspace, size_t workspace_bytes, void* stream);
+/* out = hidden * rsqrt(mean(hidden^2) + eps) * (weight + 1) per row, fp32 (a model's final norm,
+ * model/qwen35_moe_dflash/fused/model.py:206-212); out may be hidden. */
+int dflash_rms_norm(const float* hidden, int64_t tokens, int64_t hidden_size, const float* weight, float eps, float* out,
+                    void* stream);
 /* Commit of a prefix that ends inside a chunk: the state after the chunk's first `accepted` (1..16) tokens, from the
  * state before the chunk and its rows of the mixer's keys, u (head_stride elements per head, 128 per token) and cum
  * (cum_stride per head); and columns [first, first + 3) of the window bf16 [channels][pitch] as the conv history. */

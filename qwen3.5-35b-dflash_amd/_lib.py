@@ -117,7 +117,8 @@ SIGNATURES = {
     "dflash_moe_w4a16_noalloc": (ctypes.c_int, [_P, _I64, _I64, _P, _P, _I64, _W4P, _W4P, _W4P, _W4P, _P, _P, _P, _P,
                                                 _P, _P, _P, _P, _P]),
     "dflash_gdn_workspace_bytes": (_SZ, [_I64, _I64, _I64, _I64]),
-    "dflash_gdn_mixer": (ctypes.c_int, [_GDNP, _P, _I64, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _SZ, _P]),
+    "dflash_gdn_mixer": (ctypes.c_int, [_GDNP, _P, _I64, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _SZ, _P]),
+    "dflash_rms_norm": (ctypes.c_int, [_P, _I64, _I64, _P, ctypes.c_float, _P, _P]),
     "dflash_gdn_commit": (ctypes.c_int, [_P, _P, _P, _P, _I64, _I64, _I64, _I64, _P, _P, _I64, _I64, _I64, _P, _P]),
     "dflash_attention_workspace_bytes": (_SZ, [_I64, _I64, _I64, _I64, _I64]),
     "dflash_attention_mixer": (ctypes.c_int, [_ATTNP, _P, _I64, _I64, _P, _P, _I64, _P, _P, _P, _SZ, _P]),

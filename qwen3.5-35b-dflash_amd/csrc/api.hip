@@ -847,7 +847,7 @@ size_t dflash_gdn_workspace_bytes(int64_t tokens, int64_t hidden_size, int64_t k
 }
 
 int dflash_gdn_mixer(const dflash_gdn* g, const float* hidden, int64_t tokens, const void* history, const float* state,
-                     float* mid, void* normed, void* window, float* states, float* keys, float* u, float* cum,
+                     float* mid, void* normed, void* window, void* tail, float* states, float* keys, float* u, float* cum,
                      float* core, void* workspace, size_t workspace_bytes, void* stream) {
   try {
     if (!g) return fail(DFLASH_ERR_INVALID_ARGUMENT, "gdn: descriptor is NULL");
@@ -862,7 +862,7 @@ int dflash_gdn_mixer(const dflash_gdn* g, const float* hidden, int64_t tokens, c
     if (int r = check_w4(&g->out_proj, "gdn out_proj", 1, H, vw)) return r;
     if (T == 0) return DFLASH_OK;
     if (!mixer_args_aligned({g->input_norm, g->post_norm, g->norm, g->conv, hidden, history, state, mid, normed, window,
-                             states, keys, u, cum, core}) || !g->a_log || !g->dt_bias)
+                             tail, states, keys, u, cum, core}) || !g->a_log || !g->dt_bias)
       return fail(DFLASH_ERR_INVALID_ARGUMENT, "gdn: NULL or misaligned pointer");
     const GdnLayout L = gdn_layout(T, H, Hk, Hv);
     if (!workspace || workspace_bytes < L.total || !aligned16(workspace))
@@ -885,6 +885,7 @@ int dflash_gdn_mixer(const dflash_gdn* g, const float* hidden, int64_t tokens, c
     p.eps = g->eps;
     p.state = state;
     p.window = static_cast<uint16_t*>(window);
+    p.tail = static_cast<uint16_t*>(tail);
     p.keys = keys;
     p.u = u;
     p.cum = cum;
@@ -912,6 +913,19 @@ int dflash_gdn_mixer(const dflash_gdn* g, const float* hidden, int64_t tokens, c
   } catch (...) {
     return fail(DFLASH_ERR_HIP, "unexpected host exception");
   }
+}
+
+int dflash_rms_norm(const float* hidden, int64_t tokens, int64_t hidden_size, const float* weight, float eps, float* out,
+                    void* stream) {
+  if (tokens < 0 || tokens > (1 << 24)) return fail(DFLASH_ERR_UNSUPPORTED, "rms_norm: tokens must be in [0, 2^24]");
+  if (hidden_size <= 0 || hidden_size % 4 || hidden_size > dflash::kMaxNormWidth)
+    return fail(DFLASH_ERR_UNSUPPORTED, "rms_norm: hidden_size must be a multiple of 4, at most 8192");
+  if (tokens == 0) return DFLASH_OK;
+  if (!mixer_args_aligned({hidden, weight, out}))
+    return fail(DFLASH_ERR_INVALID_ARGUMENT, "rms_norm: NULL or misaligned pointer");
+  dflash::launch_norm_f32(hidden, weight, eps, static_cast<int>(tokens), static_cast<int>(hidden_size), out,
+                          static_cast<hipStream_t>(stream));
+  return launch_status("rms_norm");
 }
 
 int dflash_gdn_commit(const float* state, const float* keys, const float* u, const float* cum, int64_t head_stride,

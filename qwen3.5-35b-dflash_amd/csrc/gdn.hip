@@ -28,11 +28,12 @@ constexpr int kRow = kD + 4;     // LDS row pitch of a 128-wide fp32 row
 __device__ __forceinline__ float silu_f32(float x) { return x / (1.0f + expf(-x)); }
 
 // ------------------------------------------------------------------ residual add + RMS norm
-// One workgroup per row.  mid = hidden + mixed (when mixed is given), normed = bf16(mid * rsqrt(mean mid^2
-// + eps) * (w + 1)).  Bound by latency at the block sizes of a decode or verify call (one row is 8 KB);
+// One workgroup per row.  mid = hidden + mixed (when mixed is given), normed = mid * rsqrt(mean mid^2 + eps) * (w + 1),
+// bf16, or fp32 (kF32: a model's final norm, one launch in place of seven).  Bound by latency at the block sizes of a decode or verify call (one row is 8 KB);
 // one launch (T = 16: 3.2 us) in place of eight elementwise and reduction launches (25 us).
+template <bool kF32>
 __global__ __launch_bounds__(512) void add_norm_kernel(const float* hidden, const uint16_t* mixed, const float* w,
-                                                       float eps, int H, float* mid, uint16_t* normed) {
+                                                       float eps, int H, float* mid, void* normed) {
   __shared__ float part[8];
   const int64_t row = blockIdx.x;
   const int tid = threadIdx.x;
@@ -65,12 +66,18 @@ __global__ __launch_bounds__(512) void add_norm_kernel(const float* hidden, cons
     const int c = 4 * tid + 2048 * i;
     if (c < H) {
       const float4 g = *reinterpret_cast<const float4*>(w + c);
-      ushort4 o;
-      o.x = f32_to_bf16(v[i].x * inv * (g.x + 1.0f));
-      o.y = f32_to_bf16(v[i].y * inv * (g.y + 1.0f));
-      o.z = f32_to_bf16(v[i].z * inv * (g.z + 1.0f));
-      o.w = f32_to_bf16(v[i].w * inv * (g.w + 1.0f));
-      *reinterpret_cast<ushort4*>(normed + row * H + c) = o;
+      const float4 y = make_float4(v[i].x * inv * (g.x + 1.0f), v[i].y * inv * (g.y + 1.0f), v[i].z * inv * (g.z + 1.0f),
+                                   v[i].w * inv * (g.w + 1.0f));
+      if constexpr (kF32) {
+        *reinterpret_cast<float4*>(static_cast<float*>(normed) + row * H + c) = y;
+      } else {
+        ushort4 o;
+        o.x = f32_to_bf16(y.x);
+        o.y = f32_to_bf16(y.y);
+        o.z = f32_to_bf16(y.z);
+        o.w = f32_to_bf16(y.w);
+        *reinterpret_cast<ushort4*>(static_cast<uint16_t*>(normed) + row * H + c) = o;
+      }
     }
   }
 }
@@ -205,7 +212,11 @@ __global__ __launch_bounds__(1024) void gdn_chunk_kernel(GdnParams p) {
     for (int s = 0; s < 3; ++s)
       if (s == 2 || blockIdx.y == 0)
         for (int c = 2 * (wave - 4) + (lane >> 5); c < kD; c += 24)
-          if (in) p.window[(base[s] + c) * wp + t0 + t] = raw[s][t][c];
+          if (in) {
+            p.window[(base[s] + c) * wp + t0 + t] = raw[s][t][c];
+            // the window's last three columns are also the conv history after the whole block
+            if (t0 + t >= p.T) p.tail[(base[s] + c) * (kTaps - 1) + t0 + t - p.T] = raw[s][t][c];
+          }
   }
   lds_barrier();
 
@@ -418,7 +429,11 @@ __global__ __launch_bounds__(256) void gdn_commit_kernel(const float* state, con
 
 void launch_add_norm(const float* hidden, const uint16_t* mixed, const float* w, float eps, int T, int H, float* mid,
                      uint16_t* normed, hipStream_t stream) {
-  hipLaunchKernelGGL(add_norm_kernel, dim3(T), dim3(512), 0, stream, hidden, mixed, w, eps, H, mid, normed);
+  hipLaunchKernelGGL(add_norm_kernel<false>, dim3(T), dim3(512), 0, stream, hidden, mixed, w, eps, H, mid, normed);
+}
+
+void launch_norm_f32(const float* hidden, const float* w, float eps, int T, int H, float* normed, hipStream_t stream) {
+  hipLaunchKernelGGL(add_norm_kernel<true>, dim3(T), dim3(512), 0, stream, hidden, nullptr, w, eps, H, nullptr, normed);
 }
 
 void launch_gdn(const GdnParams& p, hipStream_t stream) {

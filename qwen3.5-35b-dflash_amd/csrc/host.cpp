@@ -32,6 +32,7 @@ struct Entries {
   decltype(&dflash_gdn_workspace_bytes) gdn_workspace_bytes;
   decltype(&dflash_gdn_mixer) gdn;
   decltype(&dflash_gdn_commit) commit;
+  decltype(&dflash_rms_norm) rms_norm;
   decltype(&dflash_attention_workspace_bytes) attention_workspace_bytes;
   decltype(&dflash_attention_mixer) attention;
 } g_entry;
@@ -254,8 +255,9 @@ PyObject* gdn(PyObject*, PyObject* const* a, Py_ssize_t n) {
   g.key_heads = hk;
   g.value_heads = hv;
   g.eps = static_cast<float>(PyFloat_AS_DOUBLE(a[12]));
-  at::Tensor o[8] = {make({t, h}, at::kFloat, device), make({t, h}, at::kBFloat16, device),
-                     make({1, width, 3 + t}, at::kBFloat16, device), make({(t + 15) / 16, 1, hv, 128, 128}, at::kFloat, device),
+  at::Tensor o[9] = {make({t, h}, at::kFloat, device), make({t, h}, at::kBFloat16, device),
+                     make({1, width, 3 + t}, at::kBFloat16, device), make({1, width, 3}, at::kBFloat16, device),
+                     make({(t + 15) / 16, 1, hv, 128, 128}, at::kFloat, device),
                      make({1, hv, t, 128}, at::kFloat, device), make({1, hv, t, 128}, at::kFloat, device),
                      make({1, hv, t}, at::kFloat, device), make({1, hv, t, 128}, at::kFloat, device)};
   const auto f = [&](int i) { return static_cast<float*>(o[i].data_ptr()); };
@@ -264,13 +266,33 @@ PyObject* gdn(PyObject*, PyObject* const* a, Py_ssize_t n) {
   int status;
   Py_BEGIN_ALLOW_THREADS
   status = g_entry.gdn(&g, static_cast<const float*>(x->data_ptr()), t, history->data_ptr(),
-                       static_cast<const float*>(state->data_ptr()), f(0), o[1].data_ptr(), o[2].data_ptr(), f(3), f(4), f(5),
-                       f(6), f(7), ws.data_ptr(), ws.numel(), st);
+                       static_cast<const float*>(state->data_ptr()), f(0), o[1].data_ptr(), o[2].data_ptr(), o[3].data_ptr(), f(4),
+                       f(5), f(6), f(7), f(8), ws.data_ptr(), ws.numel(), st);
   Py_END_ALLOW_THREADS
   if (status) Py_RETURN_NONE;
-  PyObject* r = PyTuple_New(8);
-  for (int i = 0; r && i < 8; ++i) PyTuple_SET_ITEM(r, i, THPVariable_Wrap(std::move(o[i])));
+  PyObject* r = PyTuple_New(9);
+  for (int i = 0; r && i < 9; ++i) PyTuple_SET_ITEM(r, i, THPVariable_Wrap(std::move(o[i])));
   return r;
+  END_HANDLE_TH_ERRORS
+}
+
+// rms_norm(hidden, weight, eps)
+PyObject* rms_norm(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  if (!want(n, 3)) return nullptr;
+  const at::Tensor* x = residual_stream(a[0]);
+  const at::Tensor* w = x ? exactly(a[1], at::kFloat, {x->size(1)}, x->device()) : nullptr;
+  if (!w || !PyFloat_CheckExact(a[2]) || (w->requires_grad() && c10::GradMode::is_enabled())) Py_RETURN_NONE;
+  at::Tensor out = make(x->sizes(), at::kFloat, x->device());
+  void* st = stream_of(x->device());
+  int status;
+  Py_BEGIN_ALLOW_THREADS
+  status = g_entry.rms_norm(static_cast<const float*>(x->data_ptr()), x->size(0), x->size(1),
+                            static_cast<const float*>(w->data_ptr()), static_cast<float>(PyFloat_AS_DOUBLE(a[2])),
+                            static_cast<float*>(out.data_ptr()), st);
+  Py_END_ALLOW_THREADS
+  if (status) Py_RETURN_NONE;
+  return THPVariable_Wrap(std::move(out));
   END_HANDLE_TH_ERRORS
 }
 
@@ -397,6 +419,7 @@ PyObject* bind(PyObject*, PyObject* args) {
   get("dflash_gdn_workspace_bytes", g_entry.gdn_workspace_bytes);
   get("dflash_gdn_mixer", g_entry.gdn);
   get("dflash_gdn_commit", g_entry.commit);
+  get("dflash_rms_norm", g_entry.rms_norm);
   get("dflash_attention_workspace_bytes", g_entry.attention_workspace_bytes);
   get("dflash_attention_mixer", g_entry.attention);
   if (!ok) {
@@ -411,7 +434,7 @@ PyObject* bind(PyObject*, PyObject* args) {
 }
 
 #define FAST(name) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(name)), METH_FASTCALL, nullptr}
-PyMethodDef methods[] = {FAST(linear), FAST(moe), FAST(gdn), FAST(attention), FAST(commit),
+PyMethodDef methods[] = {FAST(linear), FAST(moe), FAST(gdn), FAST(attention), FAST(commit), FAST(rms_norm),
                          {"bind", bind, METH_VARARGS, nullptr}, {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "dflash_host", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 

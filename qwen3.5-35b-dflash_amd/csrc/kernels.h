@@ -303,6 +303,8 @@ constexpr int kMaxNormWidth = 8192;  // row width launch_add_norm takes (a multi
 // mid = hidden + mixed (mixed null: mid not written), normed = bf16(rms(mid) * (w + 1)); rows of H columns
 void launch_add_norm(const float* hidden, const uint16_t* mixed, const float* w, float eps, int T, int H, float* mid,
                      uint16_t* normed, hipStream_t stream);
+// normed = rms(hidden) * (w + 1) in fp32
+void launch_norm_f32(const float* hidden, const float* w, float eps, int T, int H, float* normed, hipStream_t stream);
 struct GdnParams {
   const uint16_t* proj;    // bf16 [T][ldp]: q | k | v | z | b | a
   int ldp;
@@ -316,6 +318,7 @@ struct GdnParams {
   const float* state;      // [Hv][128][128] before the block
   // kept by the caller
   uint16_t* window;        // bf16 [C][3 + T]
+  uint16_t* tail;          // bf16 [C][3], the window's last columns
   float* keys;             // [Hv][T][128] normalised keys
   float* u;                // [Hv][T][128] delta-rule writes
   float* cum;              // [Hv][T] log decay summed inside each chunk

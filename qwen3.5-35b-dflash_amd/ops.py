@@ -158,6 +158,7 @@ class GdnMixer(NamedTuple):
     mid: torch.Tensor        # fp32 [T, H] residual after the mixer
     normed: torch.Tensor     # bf16 [T, H] its post-norm
     window: torch.Tensor     # bf16 [1, C, 3 + T]
+    tail: torch.Tensor       # bf16 [1, C, 3], its last columns
     states: torch.Tensor     # fp32 [chunks, 1, Hv, 128, 128]
     keys: torch.Tensor       # fp32 [1, Hv, T, 128]
     u: torch.Tensor          # fp32 [1, Hv, T, 128]
@@ -176,33 +177,42 @@ def gdn_mixer(hidden: torch.Tensor, history: torch.Tensor, state: torch.Tensor, 
     b16 = dict(dtype=torch.bfloat16, device=device)
     rows = (1, hv, t, 128)
     r = GdnMixer(torch.empty((t, h), **f32), torch.empty((t, h), **b16),
-                 torch.empty((1, conv.shape[0], 3 + t), **b16),
+                 torch.empty((1, conv.shape[0], 3 + t), **b16), torch.empty((1, conv.shape[0], 3), **b16),
                  torch.empty(((t + 15) // 16, 1, hv, 128, 128), **f32), torch.empty(rows, **f32),
                  torch.empty(rows, **f32), torch.empty((1, hv, t), **f32), torch.empty(rows, **f32))
     desc = _lib.GdnDesc(_desc(in_proj), _desc(out_proj), input_norm.data_ptr(), post_norm.data_ptr(), norm.data_ptr(),
                         a_log.data_ptr(), dt_bias.data_ptr(), conv.data_ptr(), h, key_heads, hv, eps)
     ws = _workspace(_lib.load().dflash_gdn_workspace_bytes(t, h, key_heads, hv), device, None)
     _lib.call("dflash_gdn_mixer", ctypes.byref(desc), _ptr(hidden), t, _ptr(history), _ptr(state), _ptr(r.mid),
-              _ptr(r.normed), _ptr(r.window), _ptr(r.states), _ptr(r.keys), _ptr(r.u), _ptr(r.cum), _ptr(r.core),
+              _ptr(r.normed), _ptr(r.window), _ptr(r.tail), _ptr(r.states), _ptr(r.keys), _ptr(r.u), _ptr(r.cum), _ptr(r.core),
               _ptr(ws), ws.numel(), _stream(device))
     return r
+
+
+def rms_norm(hidden: torch.Tensor, weight: torch.Tensor, eps: float) -> Optional[torch.Tensor]:
+    """``layers.rms_normalise(hidden, weight, eps, 1.0)`` of a plain fp32 residual ``[T, H]`` in one launch; None for other
+    forms (and where a gradient is asked for)."""
+    return _lib.host().rms_norm(hidden, weight, eps) if _plain(hidden) else None
 
 
 def gdn_mixer_plain(hidden, history, state, *, in_proj, out_proj, input_norm, post_norm, norm, a_log, dt_bias, conv,
                     key_heads, eps) -> Optional[GdnMixer]:
     """:func:`gdn_mixer` of arguments :func:`gdn_mixer_fits` accepts, both in one native call; None for others."""
-    r = _plain(hidden) and _lib.host().gdn(hidden, history, state, in_proj, out_proj, input_norm, post_norm, norm, a_log,
-                                           dt_bias, conv, key_heads, eps)
-    return GdnMixer(*r) if r else None
+    if not _plain(hidden):
+        return None
+    r = _lib.host().gdn(hidden, history, state, in_proj, out_proj, input_norm, post_norm, norm, a_log, dt_bias, conv,
+                        key_heads, eps)
+    return None if r is None else GdnMixer(*r)
 
 
 def attention_mixer_plain(hidden, keys, values, position, *, in_proj, out_proj, input_norm, post_norm, q_norm, k_norm,
                           inv_freq, heads, kv_heads, head_dim, eps) -> Optional[tuple]:
     """:func:`attention_mixer` of arguments :func:`attention_mixer_fits` accepts, both in one native call; None for
     others."""
-    r = _plain(hidden) and _lib.host().attention(hidden, keys, values, position, in_proj, out_proj, input_norm, post_norm,
-                                                 q_norm, k_norm, inv_freq, heads, kv_heads, head_dim, eps)
-    return r or None
+    if not _plain(hidden):
+        return None
+    return _lib.host().attention(hidden, keys, values, position, in_proj, out_proj, input_norm, post_norm, q_norm, k_norm,
+                                 inv_freq, heads, kv_heads, head_dim, eps)
 
 
 def _as(t, dtype: torch.dtype, shape: tuple, device: torch.device) -> bool:

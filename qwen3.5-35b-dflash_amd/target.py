@@ -184,6 +184,7 @@ class GdnPending(NamedTuple):
     window: Tensor              # bf16 [1, C, K-1+T]: conv history followed by the block's columns
     state: Tensor               # fp32 [1, Hv, Dk, Dv]: recurrent state before the block
     chunks: list                # layers.DeltaChunk per 16 tokens
+    tail: Optional[Tensor] = None   # bf16 [1, C, K-1]: the window's last columns, a tensor of its own
 
 
 class Pending(NamedTuple):
@@ -322,10 +323,11 @@ class TargetModel:
             r = ops.gdn_mixer(hidden, conv_hist, state, **args)
         n = layers.CHUNK
         if hidden.shape[0] <= n:
-            return r.mid, r.normed, GdnPending(r.window, state, [layers.DeltaChunk(r.core, r.states[0], r.keys, r.u, r.cum)])
+            return r.mid, r.normed, GdnPending(r.window, state, [layers.DeltaChunk(r.core, r.states[0], r.keys, r.u, r.cum)],
+                                                  r.tail)
         chunks = [layers.DeltaChunk(*f) for f in zip(r.core.split(n, 2), r.states.unbind(0), r.keys.split(n, 2),
                                                      r.u.split(n, 2), r.cum.split(n, 2))]
-        return r.mid, r.normed, GdnPending(r.window, state, chunks)
+        return r.mid, r.normed, GdnPending(r.window, state, chunks, r.tail)
 
     def _attention_kernels(self, hidden: Tensor, lw: LayerWeights, keys: Tensor, values: Tensor, pos: int):
         """The mixer half of an attention layer on the HIP kernels: ``(mid, moe input)``, or ``None`` when the
@@ -381,7 +383,9 @@ class TargetModel:
             gdn.append(p)
             if i in self.feature_layers:
                 feats.append(hidden)
-        final = layers.rms_normalise(hidden, self.w.final_norm, self.config.rms_eps, 1.0)
+        final = ops.rms_norm(hidden, self.w.final_norm, self.config.rms_eps)
+        if final is None:
+            final = layers.rms_normalise(hidden, self.w.final_norm, self.config.rms_eps, 1.0)
         best = None
         if top1:
             logits = ops.qlinear(final.to(torch.bfloat16), self.w.lm_head)
@@ -416,7 +420,8 @@ class TargetModel:
                     state.recurrent[i], state.conv[i] = done
                     continue
                 s = layers.state_after(s, ch.keys, ch.u, ch.cum, rest)
-            state.conv[i] = p.window[:, :, accepted:accepted + keep].clone()
+            whole_block = accepted == pending.tokens and p.tail is not None
+            state.conv[i] = p.tail if whole_block else p.window[:, :, accepted:accepted + keep].clone()
             # a state of its own: not the one before the block, nor a view that keeps every chunk's alive
             whole = s.untyped_storage().nbytes() == s.nbytes
             state.recurrent[i] = s if s is not p.state and whole else s.clone()

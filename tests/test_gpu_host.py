@@ -112,3 +112,29 @@ def test_calls_run_on_the_current_stream(pkg, device):
         y = pkg.ops.qlinear(late, w)
     stream.synchronize()
     assert torch.equal(y, want)
+
+
+@pytest.mark.parametrize("tokens,hidden", [(1, 512), (3, 2048), (70, 8192)])
+def test_rms_norm(pkg, device, tokens, hidden):
+    """The one-launch final norm against the norm in 64 bits: a few fp32 roundings (2^-24 each)."""
+    x = torch.randn((tokens, hidden), device=device) * 3
+    w = torch.randn((hidden,), device=device)
+    y = pkg.ops.rms_norm(x, w, 1e-6)
+    want = x.double() * (x.double().square().mean(-1, keepdim=True) + 1e-6).rsqrt() * (w.double() + 1)
+    assert ((y - want).norm() / want.norm()).item() <= 3e-7
+    assert pkg.ops.rms_norm(x.to(torch.bfloat16), w, 1e-6) is None
+    assert pkg.ops.rms_norm(x[:, ::2], w[::2], 1e-6) is None
+    assert pkg.ops.rms_norm(x.requires_grad_(), w, 1e-6) is None
+
+
+@pytest.mark.parametrize("tokens", [1, 2, 15, 16, 17, 18, 19, 35])
+def test_commit_of_a_whole_block_takes_the_windows_tail(pkg, device, tokens):
+    """The conv history after a whole block, also where the last chunk holds fewer tokens than the taps."""
+    c = pkg.target.small_config(("linear_attention",))
+    layout = "tiled" if tokens <= 32 else "portable"
+    model = pkg.target.TargetModel(pkg.target.random_weights(c, seed=3, device=device, layout=layout), capacity=80)
+    state = model.synthetic_context(9, seed=4)
+    _, pending = model.layer(0, torch.randn((tokens, c.hidden), device=device), state)
+    model.commit(state, pkg.target.Pending(9, tokens, [pending]), tokens)
+    assert torch.equal(state.conv[0], pending.window[:, :, tokens:])
+    assert state.conv[0].untyped_storage().nbytes() == state.conv[0].nbytes
