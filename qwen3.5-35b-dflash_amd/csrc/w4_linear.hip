@@ -12,7 +12,7 @@
 //       8192 441 -> 352 us, 2048 x 12352 x 2048 118 -> 113 us; 96-row tiles at two a CU 398 and 121 us).
 //       The MFMAs accumulate into u, the running sum in units of the current group's scale: u is rescaled by
 //       s_prev / s at each k-block in the FMA that adds the offset term, which saves a second accumulator set.
-//       Scales count as at least 2^-64 in magnitude there.
+//       A wave that meets a scale which is no unit (zero, tiny, huge, not finite) takes its columns once more without.
 //       Bound by power: in the k-loop a workgroup takes 1509 cycles a k-block where the matrix core needs 1024, at a clock
 //       that falls from 2.4 to about 1.6 GHz.  2048 x 12352 x 2048: 113 us, 0.92 PFLOP/s (bf16 library product of that
 //       size 102 us; the 16-column streaming kernel that served these sizes before 267 us; 105 us among other calls).
@@ -155,6 +155,9 @@ struct Weights {
 
 // ------------------------------------------------------------------ tiles
 constexpr int kSub = 2;  // 32-row subtiles of a tile
+// Scales a running sum may be in units of: the sum of a column whose scales lie in between stays finite in any of their
+// units while its products' sum is below 2^95.
+constexpr float kMinUnit = 0x1p-24f, kMaxUnit = 0x1p8f;
 
 typedef __attribute__((address_space(3))) void* lds_ptr;
 // 16 bytes a lane straight into LDS (lane l at dst + 16 l)
@@ -194,6 +197,7 @@ __global__ __launch_bounds__(256, 3) void w4_linear_tile_kernel(LinearParams p) 
 
   f32x16 u[kSub][2];
   float s_cur[2], s_last[2], ratio[2];  // the group scale u is in units of, the one before, and their quotient
+  bool odd = false;                     // some column of the wave has a scale that is no unit (in all lanes)
 #pragma unroll
   for (int f = 0; f < 2; ++f) {
     s_cur[f] = 0.f;
@@ -217,8 +221,8 @@ __global__ __launch_bounds__(256, 3) void w4_linear_tile_kernel(LinearParams p) 
     __builtin_amdgcn_sched_barrier(0);
   };
   auto set_scale = [&](int kb, int f, uint32_t bits) {
-    float s = scale_value<ScaleT>(bits);
-    if (__builtin_fabsf(s) < 0x1p-64f) s = __builtin_copysignf(0x1p-64f, s);  // NaN passes through
+    const float s = scale_value<ScaleT>(bits), mag = __builtin_fabsf(s);
+    odd |= __builtin_amdgcn_ballot_w64(!(mag >= kMinUnit && mag <= kMaxUnit)) != 0;  // NaN too
     ratio[f] = weights.gshift && (kb & 1) ? 1.0f : s_cur[f] * __builtin_amdgcn_rcpf(s);  // the same group still
     s_last[f] = s_cur[f];
     s_cur[f] = s;
@@ -298,6 +302,41 @@ __global__ __launch_bounds__(256, 3) void w4_linear_tile_kernel(LinearParams p) 
   }
 
   __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): no load may land in LDS once the stages are reused
+
+  if (odd) {
+    // once more without units: every k-block's sums times its scale, operands straight from memory (u is free here, so
+    // this costs the loop above no registers; a second accumulator there spilled 355 of them)
+#pragma unroll
+    for (int f = 0; f < 2; ++f) {
+      s_last[f] = 1.0f;
+#pragma unroll
+      for (int ms = 0; ms < kSub; ++ms) u[ms][f] = zero16();
+    }
+#pragma unroll 1
+    for (int kb = 0; kb < nkb; ++kb) {
+      uint4 w[2][2];
+      uint32_t sc[2];
+      weights.load(kb, w, sc);
+#pragma unroll
+      for (int ms = 0; ms < kSub; ++ms) {
+        const int at = min(ms, live - 1) * nkb + kb;
+#pragma unroll
+        for (int f = 0; f < 2; ++f) {
+          f32x16 acc;
+#pragma unroll
+          for (int g = 0; g < 4; ++g) {
+            const f32x4 start = __builtin_bit_cast(f32x4, buf_load16(nrs, h * 16, at * 128 + g * 32));
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[4 * g + e] = start[e];
+          }
+#pragma unroll
+          for (int j = 0; j < 8; ++j)
+            acc = mfma32(buf_load16(ars, lane * 16, at * 8192 + j * 1024), dequant24(word(w[f][j >> 2], j & 3)), acc);
+          u[ms][f] += scale_value<ScaleT>(sc[f]) * acc;
+        }
+      }
+    }
+  }
 
   // lane: rows 32 ms + 8 (i / 4) + 4 h + i % 4 of columns col0 + 32 f + r
   if (p.y_f32) {
