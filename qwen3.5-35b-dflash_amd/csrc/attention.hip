@@ -185,7 +185,8 @@ __global__ __launch_bounds__(256, 1) void attn_split_kernel(AttnParams p) {
     mc = fmaxf(mc, __shfl_xor(mc, 16, 64));
     mc = fmaxf(mc, __shfl_xor(mc, 32, 64));
     const float mn = fmaxf(m, mc);
-    // a row that has seen no key yet keeps weight 0 (its maximum is -inf, as is every score)
+    // a row that has seen no key yet keeps weight 0 (its maximum is -inf, as is every score); a NaN score, which the
+    // maximum skips, makes l and o NaN, and so they stay
     const float corr = mn == -__builtin_inff() ? 1.f : expf(m - mn);
     float sum = 0.f;
 #pragma unroll
@@ -219,7 +220,8 @@ __global__ __launch_bounds__(256, 1) void attn_split_kernel(AttnParams p) {
         o[c] = mfma16x16x32(__builtin_bit_cast(uint4, a), __builtin_bit_cast(uint4, pf[b]), o[c]);
     }
   }
-  // merge the four waves: each scales its sums to the workgroup's maximum
+  // merge the four waves: each scales its sums to the workgroup's maximum (a wave without keys has sums of 0, not
+  // only a maximum of -inf: with scores that are all NaN its sums are NaN and stay in)
   if (kq == 0) {
     mx[wave][lr] = m;
     ls[wave][lr] = l;
@@ -245,14 +247,14 @@ __global__ __launch_bounds__(256, 1) void attn_split_kernel(AttnParams p) {
     const float mm = fmaxf(fmaxf(mx[0][tid], mx[1][tid]), fmaxf(mx[2][tid], mx[3][tid]));
     float sum = 0.f;
 #pragma unroll
-    for (int w = 0; w < 4; ++w) sum += mx[w][tid] == -__builtin_inff() ? 0.f : ls[w][tid] * expf(mx[w][tid] - mm);
+    for (int w = 0; w < 4; ++w) sum += mx[w][tid] == -__builtin_inff() ? ls[w][tid] * 0.f : ls[w][tid] * expf(mx[w][tid] - mm);
     p.ml[out_row + tid] = make_float2(mm, sum);
   }
 }
 
 // One workgroup per (token, head), one dim a thread.  Each wave reads every split's maximum and sum at once, a split a
 // lane (one after the other they were most of this kernel's time), and the partial rows follow eight at a time.  Splits
-// that hold no key of the row (maximum -inf, partial row never written) are left out.
+// that hold no key of the row (sum 0, partial row maybe never written) are left out.
 constexpr int kMaxSplits = 256;
 template <int D>
 __global__ __launch_bounds__(D) void attn_combine_kernel(AttnParams p) {
@@ -275,7 +277,7 @@ __global__ __launch_bounds__(D) void attn_combine_kernel(AttnParams p) {
   float l = 0.f;
 #pragma unroll
   for (int i = 0; i < kPer; ++i) {
-    const bool used = v[i].x != -__builtin_inff();
+    const bool used = v[i].y != 0.f;  // a NaN sum (NaN scores) is used and makes the row NaN
     const float f = used ? expf(v[i].x - M) : -1.f;
     if (used) l += v[i].y * f;
     if (threadIdx.x < 64) fs[lane + 64 * i] = f;

@@ -114,3 +114,38 @@ def test_moe_with_the_residual_add(pkg, device, tokens, split_down):
     assert torch.equal(got, want)
     with pytest.raises(ValueError, match="residual"):
         pkg.ops.moe_w4a16_add(residual.to(torch.bfloat16), x, *banks, **args)
+
+
+def _attention_model(pkg, device, heads, kv_heads, head_dim, capacity, layout="tiled"):
+    base = pkg.target.small_config(("full_attention",))
+    c = type(base)(**{**vars(base), "heads": heads, "kv_heads": kv_heads, "head_dim": head_dim})
+    return c, pkg.target.TargetModel(pkg.target.random_weights(c, seed=9, device=device, layout=layout), capacity=capacity)
+
+
+def _mixer_and_general(model, x, state):
+    """The residual after the mixer, from the kernels and from the PyTorch form of the same layer."""
+    lw, eps = model.w.layers[0], model.config.rms_eps
+    trace, other = {}, state.clone()
+    model.layer(0, x, state, trace=trace)
+    normed = (x * (x.square().mean(-1, keepdim=True) + eps).rsqrt() * (lw.input_norm + 1)).to(torch.bfloat16)
+    general = x + model._attention(normed, lw, other.keys[0], other.values[0], other.position).float()
+    return trace["mid"], general
+
+
+@pytest.mark.parametrize("tokens,context,stretch", [
+    (1, 896, None), (1, 1920, None),         # the last split holds the token's own key alone
+    (1, 300, (128, 256)), (16, 1000, (128, 256)), (16, 1000, (640, 704)),     # whole splits and whole key steps
+    (5, 40, (32, 33)),
+])
+def test_attention_keeps_a_nan_key(pkg, device, tokens, context, stretch):
+    """A NaN in a visible key makes the softmax of the rows that see it NaN, wherever the key falls: a split, or a
+    wave's part of one, in which every score is NaN is not one without keys."""
+    c, model = _attention_model(pkg, device, 16, 2, 256, context + tokens + 3)
+    state = model.synthetic_context(context, seed=10)
+    if stretch is None:
+        model.w.layers[0].k_norm[3] = float("nan")       # the block's own K rows
+    else:
+        state.keys[0][:, :, stretch[0]:stretch[1], 7] = float("nan")
+    x = torch.randn((tokens, c.hidden), generator=torch.Generator().manual_seed(5)).to(device)
+    got, general = _mixer_and_general(model, x, state)
+    assert torch.isnan(general).all() and torch.isnan(got).all()
