@@ -178,7 +178,10 @@ __global__ __launch_bounds__(256, 1) void attn_split_kernel(AttnParams p) {
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const int key = j0 + 16 * b + 4 * kq + e;
-        s8[4 * b + e] = key < visible && key < k1 ? acc[0][e] + (acc[1][e] + acc[2][e]) : -__builtin_inff();
+        // with an infinity in the key the leading part alone has the score (an infinity times a part of 0 or of the other
+        // sign would make it NaN)
+        const float score = __builtin_fabsf(acc[0][e]) < __builtin_inff() ? acc[0][e] + (acc[1][e] + acc[2][e]) : acc[0][e];
+        s8[4 * b + e] = key < visible && key < k1 ? score : -__builtin_inff();
       }
     }
     float mc = fmaxf(fmaxf(fmaxf(s8[0], s8[1]), fmaxf(s8[2], s8[3])), fmaxf(fmaxf(s8[4], s8[5]), fmaxf(s8[6], s8[7])));

@@ -149,3 +149,29 @@ def test_attention_keeps_a_nan_key(pkg, device, tokens, context, stretch):
     x = torch.randn((tokens, c.hidden), generator=torch.Generator().manual_seed(5)).to(device)
     got, general = _mixer_and_general(model, x, state)
     assert torch.isnan(general).all() and torch.isnan(got).all()
+
+
+@pytest.mark.parametrize("kv_heads,group", [(4, 1), (4, 3)])
+def test_attention_over_an_infinite_key(pkg, device, kv_heads, group):
+    """A key that scores -inf has weight 0; one that scores +inf makes the row NaN, as in the softmax."""
+    c, model = _attention_model(pkg, device, kv_heads * group, kv_heads, 128, 320, layout="portable")
+    lw = model.w.layers[0]
+    x = torch.randn((1, c.hidden), generator=torch.Generator().manual_seed(6)).to(device)
+    state = model.synthetic_context(300, seed=10)
+    want, _ = _mixer_and_general(model, x, state.clone())
+    normed = (x * (x.square().mean(-1, keepdim=True) + c.rms_eps).rsqrt() * (lw.input_norm + 1)).to(torch.bfloat16)
+    q = pkg.ops.qlinear(normed, lw.mixer_in)[0, :2 * c.heads * 128].float().view(kv_heads, group, 256)[..., 64:128]
+    same = (q > 0).all(1) | (q < 0).all(1)               # a feature past the rotary ones in which a KV head's queries agree
+    assert bool(same.any(1).all())
+    feature = same.float().argmax(1)
+    sign = q[:, 0].gather(1, feature[:, None])[:, 0].sign() * (lw.q_norm[64 + feature] + 1).sign()
+    for scores, key in ((-1, 17), (-1, 299), (1, 17)):
+        bad = state.clone()
+        for h in range(kv_heads):
+            bad.keys[0][0, h, key, 64 + feature[h]] = scores * sign[h] * float("inf")
+        got, general = _mixer_and_general(model, x, bad)
+        if scores > 0:
+            assert torch.isnan(general).all() and torch.isnan(got).all()
+        else:
+            assert torch.isfinite(general).all() and not torch.equal(general, want)
+            assert metrics.compare(got.cpu() - x.cpu(), general.cpu() - x.cpu())["max_rel"] <= TOL
