@@ -9,7 +9,10 @@ from __future__ import annotations
 import ctypes
 import importlib.machinery
 import importlib.util
+import warnings
 from pathlib import Path
+
+import torch
 
 PACKAGE_DIR = Path(__file__).resolve().parent
 LIBRARY_PATH = PACKAGE_DIR / "libdflash_hip.so"
@@ -171,23 +174,29 @@ def load(path: Path = LIBRARY_PATH) -> ctypes.CDLL:
     return lib
 
 
-_HOST = None
+_HOST = None  # the module once loaded, False once it could not be
 
 
 def host():
-    """The native form of ops.py's plain calls (``csrc/host.cpp``), bound (once) to the loaded library's entries."""
+    """The native form of ops.py's plain calls (``csrc/host.cpp``), bound (once) to the loaded library's entries; None
+    where it was not built, or not for this torch: ops.py's own form of every call then serves."""
     global _HOST
     if _HOST is None:
         from .packing import PackedW4, SharedExpert
         lib = load()
-        if not HOST_PATH.is_file():
-            raise RuntimeError(f"{HOST_PATH.name} not found at {HOST_PATH}; build it with build.py")
-        loader = importlib.machinery.ExtensionFileLoader("dflash_host", str(HOST_PATH))
-        module = importlib.util.module_from_spec(importlib.util.spec_from_loader("dflash_host", loader))
-        loader.exec_module(module)
-        module.bind(PackedW4, SharedExpert, lambda name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value)
-        _HOST = module
-    return _HOST
+        try:
+            loader = importlib.machinery.ExtensionFileLoader("dflash_host", str(HOST_PATH))
+            module = importlib.util.module_from_spec(importlib.util.spec_from_loader("dflash_host", loader))
+            loader.exec_module(module)
+            if module.TORCH != torch.__version__:
+                raise ImportError(f"built for torch {module.TORCH}, not {torch.__version__}")
+            module.bind(PackedW4, SharedExpert, lambda name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value)
+            _HOST = module
+        except (ImportError, AttributeError) as error:
+            warnings.warn(f"{HOST_PATH.name} is not used ({error}); calls take their Python form, build.py builds it",
+                          RuntimeWarning, stacklevel=2)
+            _HOST = False
+    return _HOST or None
 
 
 def check(function: str, status: int) -> None:

@@ -48,8 +48,38 @@ def _host_command(output: Path) -> list:
                "/opt/rocm/include")
     return [shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden",
             f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-DUSE_ROCM=1", "-D__HIP_PLATFORM_AMD__=1",
+            f'-DDFLASH_TORCH="{torch.__version__}"',
             *(f"-I{i}" for i in include), str(PACKAGE_DIR / HOST_SOURCE), "-o", str(output), f"-L{root / 'lib'}",
             "-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip"]
+
+
+def _start(cmd: list) -> tuple:
+    return cmd, subprocess.Popen(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+
+
+def _start_host(output: Path):
+    """The compile of the host library, or None where g++ or torch is missing."""
+    try:
+        return _start(_host_command(output))
+    except (ImportError, OSError) as error:
+        print(f"{HOST_LIBRARY.name} is not built: {error}", file=sys.stderr)
+        return None
+
+
+def _finish_host(job) -> bool:
+    """Whether the host library was compiled.  Without it every call takes its Python form."""
+    if job is None:
+        return False
+    out, _ = job[1].communicate()
+    if job[1].returncode:
+        print(f"{HOST_LIBRARY.name} is not built: {' '.join(job[0])}\n{out}", file=sys.stderr)
+    return job[1].returncode == 0
+
+
+def _install(built: Path, final: Path) -> None:
+    tmp_target = final.with_suffix(".so.tmp")
+    shutil.copyfile(built, tmp_target)
+    os.replace(tmp_target, final)
 
 
 def build(verbose: bool = False, timeline: bool = False) -> Path:
@@ -62,11 +92,9 @@ def build(verbose: bool = False, timeline: bool = False) -> Path:
             obj = Path(tmp) / (Path(src).stem + ".o")
             cmd = [hipcc, *flags, "-c", str(PACKAGE_DIR / src), "-o", str(obj)]
             objects.append(obj)
-            procs.append((cmd, subprocess.Popen(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)))
-        host = None if timeline else Path(tmp) / HOST_LIBRARY.name
-        if host:
-            cmd = _host_command(host)
-            procs.append((cmd, subprocess.Popen(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)))
+            procs.append(_start(cmd))
+        host = Path(tmp) / HOST_LIBRARY.name
+        job = None if timeline else _start_host(host)
         for cmd, proc in procs:
             out, _ = proc.communicate()
             if proc.returncode:
@@ -78,11 +106,12 @@ def build(verbose: bool = False, timeline: bool = False) -> Path:
         proc = subprocess.run(link, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
         if proc.returncode:
             raise RuntimeError(f"link failed: {' '.join(link)}\n{proc.stdout}")
-        for built, final in ((staged, target), (host, HOST_LIBRARY)):
-            if built:
-                tmp_target = final.with_suffix(".so.tmp")
-                shutil.copyfile(built, tmp_target)
-                os.replace(tmp_target, final)
+        _install(staged, target)
+        if not timeline:
+            if _finish_host(job):
+                _install(host, HOST_LIBRARY)
+            else:
+                HOST_LIBRARY.unlink(missing_ok=True)  # not one of other sources or another torch
     return target
 
 

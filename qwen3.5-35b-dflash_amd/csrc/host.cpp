@@ -440,4 +440,8 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "dflash_host", nullptr, -1, methods
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit_dflash_host() { return PyModule_Create(&module); }
+PyMODINIT_FUNC PyInit_dflash_host() {
+  PyObject* m = PyModule_Create(&module);
+  if (m && PyModule_AddStringConstant(m, "TORCH", DFLASH_TORCH) < 0) Py_CLEAR(m);  // the torch it was compiled for
+  return m;
+}

@@ -122,7 +122,7 @@ def to_tiled(w: PackedW4) -> PackedW4:
 
 def _plain(x) -> bool:
     """Whether a call on ``x`` is first offered to the native form (``csrc/host.cpp``), which takes it or returns None."""
-    return type(x) is torch.Tensor and x.is_cuda
+    return type(x) is torch.Tensor and x.is_cuda and _lib.host() is not None
 
 
 def qlinear(x: torch.Tensor, weight: PackedW4, *, workspace: Optional[torch.Tensor] = None,

@@ -138,3 +138,22 @@ def test_commit_of_a_whole_block_takes_the_windows_tail(pkg, device, tokens):
     model.commit(state, pkg.target.Pending(9, tokens, [pending]), tokens)
     assert torch.equal(state.conv[0], pending.window[:, :, tokens:])
     assert state.conv[0].untyped_storage().nbytes() == state.conv[0].nbytes
+
+
+def test_calls_without_the_native_form(pkg, device, monkeypatch):
+    """Where dflash_host.so cannot be loaded the Python form serves every call, with the same bits."""
+    w, x = _weight(pkg, device, 96, 512), torch.randn((8, 512), device=device).to(torch.bfloat16)
+    c = pkg.target.small_config()
+    model = pkg.target.TargetModel(pkg.target.random_weights(c, seed=3, device=device), capacity=80)
+    ids = torch.arange(8, device=device)
+
+    def run():
+        state = model.synthetic_context(9, seed=4)
+        out = model.forward(ids, state)
+        model.commit(state, out.pending, 5)
+        return [pkg.ops.qlinear(x, w), out.top1, *(r for r in state.recurrent if r is not None)]
+    want = run()
+    monkeypatch.setattr(pkg._lib, "_HOST", False)
+    assert pkg._lib.host() is None
+    for a, b in zip(run(), want):
+        assert torch.equal(a, b)

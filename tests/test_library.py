@@ -317,3 +317,34 @@ def test_noalloc_refuses_oversized_layers_before_any_launch(pkg):
     st = lib.dflash_moe_w4a16_noalloc(p, 16, 2048, None, p, 8, ctypes.byref(gu16), ctypes.byref(dn), None, None,
                                       None, p, None, p, p, p, p, p, None)
     assert st != 0 and "above the static" not in lib.dflash_last_error().decode(), lib.dflash_last_error().decode()
+
+
+def test_library_serves_without_the_host_module(pkg, monkeypatch, tmp_path):
+    """No dflash_host.so, a broken one, or one for another torch: one warning, then ops.py's Python form."""
+    import torch
+    lib = pkg._lib
+    broken = tmp_path / "dflash_host.so"
+    broken.write_bytes(b"not a library")
+    for path, version in ((tmp_path / "missing.so", torch.__version__), (broken, torch.__version__), (lib.HOST_PATH, "0.0")):
+        with monkeypatch.context() as m:
+            m.setattr(lib, "_HOST", None)
+            m.setattr(lib, "HOST_PATH", path)
+            m.setattr(torch, "__version__", version)
+            with pytest.warns(RuntimeWarning, match="not used"):
+                assert lib.host() is None
+            assert lib.host() is None and not pkg.ops._plain(torch.zeros(1))
+    assert lib.host() is not None
+
+
+def test_build_goes_on_without_a_host_compiler(monkeypatch, tmp_path, capsys):
+    """No g++, or a compile that fails (torch's headers missing): the kernels' library is built all the same."""
+    import importlib.util
+    spec = importlib.util.spec_from_file_location("_build_under_test", ROOT / "qwen3.5-35b-dflash_amd" / "build.py")
+    builder = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(builder)
+    monkeypatch.setenv("PATH", str(tmp_path))
+    job = builder._start_host(tmp_path / "host.so")
+    assert job is None and not builder._finish_host(job)
+    assert not builder._finish_host(builder._start(["/bin/sh", "-c", "exit 1"]))
+    assert builder._finish_host(builder._start(["/bin/sh", "-c", "exit 0"]))
+    assert capsys.readouterr().err.count("is not built") == 2
