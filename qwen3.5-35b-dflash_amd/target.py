@@ -184,7 +184,9 @@ class GdnPending(NamedTuple):
     window: Tensor              # bf16 [1, C, K-1+T]: conv history followed by the block's columns
     state: Tensor               # fp32 [1, Hv, Dk, Dv]: recurrent state before the block
     chunks: list                # layers.DeltaChunk per 16 tokens
-    tail: Optional[Tensor] = None   # bf16 [1, C, K-1]: the window's last columns, a tensor of its own
+    # the conv history after the whole block, and its recurrent state where that is a tensor of its own: for the first
+    # commit of the whole block to take (later ones make their own, so that no two states share a tensor)
+    ends: Optional[list] = None
 
 
 class Pending(NamedTuple):
@@ -324,10 +326,10 @@ class TargetModel:
         n = layers.CHUNK
         if hidden.shape[0] <= n:
             return r.mid, r.normed, GdnPending(r.window, state, [layers.DeltaChunk(r.core, r.states[0], r.keys, r.u, r.cum)],
-                                                  r.tail)
+                                               [(r.tail, r.states[0])])
         chunks = [layers.DeltaChunk(*f) for f in zip(r.core.split(n, 2), r.states.unbind(0), r.keys.split(n, 2),
                                                      r.u.split(n, 2), r.cum.split(n, 2))]
-        return r.mid, r.normed, GdnPending(r.window, state, chunks, r.tail)
+        return r.mid, r.normed, GdnPending(r.window, state, chunks, [(r.tail, None)])
 
     def _attention_kernels(self, hidden: Tensor, lw: LayerWeights, keys: Tensor, values: Tensor, pos: int):
         """The mixer half of an attention layer on the HIP kernels: ``(mid, moe input)``, or ``None`` when the
@@ -405,24 +407,29 @@ class TargetModel:
             raise ValueError("accepted must be an integer in [0, block tokens]")
         if accepted == 0:
             return
-        keep = self.config.conv_kernel - 1
         for i, p in enumerate(pending.gdn):
-            if p is None:
-                continue
-            full, rest = divmod(accepted, layers.CHUNK)
-            if accepted == pending.tokens:                  # the whole block: a short last chunk ends there too
-                full, rest = len(p.chunks), 0
-            s = p.chunks[full - 1].state if full else p.state
-            if rest:
-                ch = p.chunks[full]
-                done = ops.gdn_commit(s, ch.keys, ch.u, ch.cum, rest, p.window, accepted) if keep == 3 else None
-                if done is not None:
-                    state.recurrent[i], state.conv[i] = done
-                    continue
-                s = layers.state_after(s, ch.keys, ch.u, ch.cum, rest)
-            whole_block = accepted == pending.tokens and p.tail is not None
-            state.conv[i] = p.tail if whole_block else p.window[:, :, accepted:accepted + keep].clone()
-            # a state of its own: not the one before the block, nor a view that keeps every chunk's alive
-            whole = s.untyped_storage().nbytes() == s.nbytes
-            state.recurrent[i] = s if s is not p.state and whole else s.clone()
+            if p is not None:
+                state.conv[i], state.recurrent[i] = self._committed(p, accepted, accepted == pending.tokens)
         state.position += accepted
+
+    def _committed(self, p: GdnPending, accepted: int, whole: bool) -> tuple:
+        """Conv history and recurrent state after the first ``accepted`` tokens, tensors no other state has."""
+        if whole and p.ends:
+            try:
+                conv, s = p.ends.pop()
+                return conv, p.chunks[-1].state.clone() if s is None else s
+            except IndexError:                              # another thread's commit took them
+                pass
+        full, rest = divmod(accepted, layers.CHUNK)
+        if whole and rest == 0 and p.ends is not None:      # the last chunk's own state may be an earlier commit's
+            full, rest = full - 1, layers.CHUNK
+        s = p.chunks[full - 1].state if full else p.state
+        keep = self.config.conv_kernel - 1
+        if rest:
+            ch = p.chunks[full]
+            done = ops.gdn_commit(s, ch.keys, ch.u, ch.cum, rest, p.window, accepted) if keep == 3 else None
+            if done is not None:
+                return done[1], done[0]
+            s = layers.state_after(s, ch.keys, ch.u, ch.cum, rest)
+        conv = p.window[:, :, accepted:accepted + keep].clone()
+        return conv, s if rest else s.clone()

@@ -157,3 +157,29 @@ def test_calls_without_the_native_form(pkg, device, monkeypatch):
     assert pkg._lib.host() is None
     for a, b in zip(run(), want):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("tokens,accepted", [(1, 1), (9, 9), (16, 16), (17, 17), (32, 32), (16, 5), (32, 16)])
+def test_two_commits_of_one_block_share_nothing(pkg, device, tokens, accepted):
+    """States committed from one pending record have tensors of their own: writing one in place changes neither the
+    others, also of commits that follow, nor the state before the block."""
+    c = pkg.target.small_config(("linear_attention",))
+    model = pkg.target.TargetModel(pkg.target.random_weights(c, seed=3, device=device), capacity=80)
+    state = model.synthetic_context(9, seed=4)
+    before = state.clone()
+    _, pending = model.layer(0, torch.randn((tokens, c.hidden), device=device), state)
+    conv, chunks = pending.window[:, :, accepted:accepted + 3].clone(), pending.chunks
+    want = pkg.layers.state_after(chunks[-2].state if len(chunks) > 1 else state.recurrent[0], chunks[-1].keys, chunks[-1].u,
+                                  chunks[-1].cum, accepted - 16 * (len(chunks) - 1)) if accepted == tokens else None
+    commits = []
+    for _ in range(3):
+        branch = pkg.target.TargetState(9, list(state.conv), list(state.recurrent), state.keys, state.values)
+        model.commit(branch, pkg.target.Pending(9, tokens, [pending]), accepted)
+        want = branch.recurrent[0].clone() if want is None else want
+        assert torch.equal(branch.conv[0], conv)
+        assert ((branch.recurrent[0] - want).norm() / want.norm()).item() <= 1e-6     # fp32 sums in another order
+        branch.conv[0].fill_(1)
+        branch.recurrent[0].fill_(1)
+        commits.append(branch)
+    assert len({t.untyped_storage().data_ptr() for b in commits for t in (b.conv[0], b.recurrent[0])}) == 6
+    assert torch.equal(state.conv[0], before.conv[0]) and torch.equal(state.recurrent[0], before.recurrent[0])
