@@ -167,7 +167,11 @@ def test_two_commits_of_one_block_share_nothing(pkg, device, tokens, accepted):
     model = pkg.target.TargetModel(pkg.target.random_weights(c, seed=3, device=device), capacity=80)
     state = model.synthetic_context(9, seed=4)
     before = state.clone()
-    _, pending = model.layer(0, torch.randn((tokens, c.hidden), device=device), state)
+    x = torch.randn((tokens, c.hidden), generator=torch.Generator().manual_seed(tokens)).to(device)
+    _, pending = model.layer(0, x, state)
+    # states rebuilt from the record differ by fp32 sums in another order and by decays e^(G_j - G_s) of log decays held
+    # in fp32, each 2^-24 |G| off
+    bound = 1e-6 + 2.0 ** -23 * pending.chunks[-1].cum.abs().max().item()
     conv, chunks = pending.window[:, :, accepted:accepted + 3].clone(), pending.chunks
     want = pkg.layers.state_after(chunks[-2].state if len(chunks) > 1 else state.recurrent[0], chunks[-1].keys, chunks[-1].u,
                                   chunks[-1].cum, accepted - 16 * (len(chunks) - 1)) if accepted == tokens else None
@@ -177,7 +181,7 @@ def test_two_commits_of_one_block_share_nothing(pkg, device, tokens, accepted):
         model.commit(branch, pkg.target.Pending(9, tokens, [pending]), accepted)
         want = branch.recurrent[0].clone() if want is None else want
         assert torch.equal(branch.conv[0], conv)
-        assert ((branch.recurrent[0] - want).norm() / want.norm()).item() <= 1e-6     # fp32 sums in another order
+        assert ((branch.recurrent[0] - want).norm() / want.norm()).item() <= bound
         branch.conv[0].fill_(1)
         branch.recurrent[0].fill_(1)
         commits.append(branch)
