@@ -49,6 +49,11 @@ const at::Tensor* tensor(PyObject* o) {
   return &t;
 }
 
+// ops._tracked: a gradient is asked for, or a forward-mode tangent is carried
+bool tracked(const at::Tensor& t) {
+  return (t.requires_grad() && c10::GradMode::is_enabled()) || t.unsafeGetTensorImpl()->_fw_grad(0, t).defined();
+}
+
 // What ops._as accepts: this dtype, shape and device, contiguous, 16-byte aligned.
 const at::Tensor* exactly(PyObject* o, at::ScalarType dtype, at::IntArrayRef shape, at::Device device) {
   const at::Tensor* t = tensor(o);
@@ -176,7 +181,7 @@ PyObject* moe(PyObject*, PyObject* const* a, Py_ssize_t n) {
       Py_RETURN_NONE;
   }
   const at::Tensor* residual = nullptr;
-  if (a[7] != Py_None && !(residual = exactly(a[7], at::kFloat, {t, h}, device))) Py_RETURN_NONE;
+  if (a[7] != Py_None && (!(residual = exactly(a[7], at::kFloat, {t, h}, device)) || tracked(*residual))) Py_RETURN_NONE;
   at::Tensor ws;
   const size_t need = g_entry.moe_workspace_bytes(t, h, gu.rows / 2, e, k, gu.group_size, shared);
   if (!workspace_of(a[6], need, device, &ws)) Py_RETURN_NONE;
@@ -211,7 +216,7 @@ PyObject* moe(PyObject*, PyObject* const* a, Py_ssize_t n) {
 const at::Tensor* residual_stream(PyObject* o) {
   const at::Tensor* t = plain_state() ? tensor(o) : nullptr;
   if (!t || t->dim() != 2 || !exactly(o, at::kFloat, t->sizes(), t->device()) || t->size(0) < 1 || t->size(0) > 1 << 19 ||
-      t->size(1) % 512 || t->size(1) < 512 || t->size(1) > 8192 || (t->requires_grad() && c10::GradMode::is_enabled()))
+      t->size(1) % 512 || t->size(1) < 512 || t->size(1) > 8192 || tracked(*t))
     return nullptr;
   return t;
 }
@@ -242,7 +247,8 @@ PyObject* gdn(PyObject*, PyObject* const* a, Py_ssize_t n) {
                    *conv = exactly(a[10], at::kBFloat16, {width, 1, 4}, device);
   dflash_gdn g{};
   if (!history || !state || !input_norm || !post_norm || !norm || !dt_bias || !conv ||
-      !exactly(a[8], at::kFloat, {hv}, device) || !matrix(a[3], width + 128 * hv + 2 * hv, h, device, &g.in_proj) ||
+      tracked(*history) || tracked(*state) || tracked(*input_norm) || tracked(*post_norm) || tracked(*norm) ||
+      tracked(*dt_bias) || tracked(*conv) || tracked(*a_log) || !exactly(a[8], at::kFloat, {hv}, device) || !matrix(a[3], width + 128 * hv + 2 * hv, h, device, &g.in_proj) ||
       !matrix(a[4], h, 128 * hv, device, &g.out_proj))
     Py_RETURN_NONE;
   g.input_norm = static_cast<const float*>(input_norm->data_ptr());
@@ -282,7 +288,7 @@ PyObject* rms_norm(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (!want(n, 3)) return nullptr;
   const at::Tensor* x = residual_stream(a[0]);
   const at::Tensor* w = x ? exactly(a[1], at::kFloat, {x->size(1)}, x->device()) : nullptr;
-  if (!w || !PyFloat_CheckExact(a[2]) || (w->requires_grad() && c10::GradMode::is_enabled())) Py_RETURN_NONE;
+  if (!w || !PyFloat_CheckExact(a[2]) || tracked(*w)) Py_RETURN_NONE;
   at::Tensor out = make(x->sizes(), at::kFloat, x->device());
   void* st = stream_of(x->device());
   int status;
@@ -327,7 +333,8 @@ PyObject* attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
                    *q_norm = exactly(a[8], at::kFloat, {d}, device), *k_norm = exactly(a[9], at::kFloat, {d}, device);
   dflash_attention g{};
   if (!exactly(a[1], at::kBFloat16, cache, device) || !values || !input_norm || !post_norm || !q_norm || !k_norm ||
-      !exactly(a[10], at::kFloat, {half}, device) || !matrix(a[4], 2 * (heads + kv) * d, h, device, &g.in_proj) ||
+      tracked(*keys) || tracked(*values) || tracked(*input_norm) || tracked(*post_norm) || tracked(*q_norm) ||
+      tracked(*k_norm) || tracked(*inv_freq) || !exactly(a[10], at::kFloat, {half}, device) || !matrix(a[4], 2 * (heads + kv) * d, h, device, &g.in_proj) ||
       !matrix(a[5], h, heads * d, device, &g.out_proj))
     Py_RETURN_NONE;
   g.input_norm = static_cast<const float*>(input_norm->data_ptr());
@@ -375,7 +382,8 @@ PyObject* commit(PyObject*, PyObject* const* a, Py_ssize_t n) {
       cum->sizes() != keys->sizes().slice(0, 3) || !f32(keys) || !f32(u) || !f32(cum) || keys->stride(2) != 128 ||
       keys->stride(3) != 1 || u->strides() != keys->strides() || cum->stride(2) != 1 ||
       window->scalar_type() != at::kBFloat16 || window->dim() != 3 || window->size(0) != 1 || window->device() != device ||
-      !window->is_contiguous() || first + 3 > window->size(2)) {
+      !window->is_contiguous() || first + 3 > window->size(2) || tracked(*state) || tracked(*keys) || tracked(*u) ||
+      tracked(*cum) || tracked(*window)) {
     PyErr_Clear();
     Py_RETURN_NONE;
   }

@@ -13,6 +13,7 @@ import ctypes
 from typing import NamedTuple, Optional
 
 import torch
+from torch.autograd import forward_ad
 
 from . import _lib
 from .packing import PackedW4, SharedExpert
@@ -191,7 +192,7 @@ def gdn_mixer(hidden: torch.Tensor, history: torch.Tensor, state: torch.Tensor, 
 
 def rms_norm(hidden: torch.Tensor, weight: torch.Tensor, eps: float) -> Optional[torch.Tensor]:
     """``layers.rms_normalise(hidden, weight, eps, 1.0)`` of a plain fp32 residual ``[T, H]`` in one launch; None for other
-    forms (and where a gradient is asked for)."""
+    forms (and where autograd follows it)."""
     return _lib.host().rms_norm(hidden, weight, eps) if _plain(hidden) else None
 
 
@@ -221,6 +222,13 @@ def _as(t, dtype: torch.dtype, shape: tuple, device: torch.device) -> bool:
             and t.is_contiguous() and t.data_ptr() % 16 == 0)
 
 
+def _tracked(*tensors) -> bool:
+    """Whether autograd follows any of them (a gradient is asked for, or it carries a forward-mode tangent): the kernels
+    drop both, so such calls take the PyTorch form."""
+    return ((torch.is_grad_enabled() and any(t.requires_grad for t in tensors))
+            or any(forward_ad.unpack_dual(t).tangent is not None for t in tensors))
+
+
 def _matrix(w, rows: int, cols: int, device: torch.device) -> bool:
     """Whether ``w`` is a valid packed matrix of this size on this device."""
     if not isinstance(w, PackedW4) or w.packed.ndim != 2 or (w.rows, w.cols) != (rows, cols):
@@ -231,17 +239,16 @@ def _matrix(w, rows: int, cols: int, device: torch.device) -> bool:
 
 def _residual(hidden: torch.Tensor) -> bool:
     """Whether the mixer kernels take this residual: fp32 ``[T, H]`` as it lies, at least one token, H they can
-    normalise, and no gradient asked for."""
+    normalise."""
     return (_as(hidden, torch.float32, hidden.shape, hidden.device) and hidden.is_cuda and hidden.ndim == 2
-            and 1 <= hidden.shape[0] <= 1 << 19 and hidden.shape[1] % 512 == 0 and 512 <= hidden.shape[1] <= 8192
-            and not (hidden.requires_grad and torch.is_grad_enabled()))
+            and 1 <= hidden.shape[0] <= 1 << 19 and hidden.shape[1] % 512 == 0 and 512 <= hidden.shape[1] <= 8192)
 
 
 def gdn_mixer_fits(hidden: torch.Tensor, history: torch.Tensor, state: torch.Tensor, *, in_proj: PackedW4,
                    out_proj: PackedW4, input_norm: torch.Tensor, post_norm: torch.Tensor, norm: torch.Tensor,
                    a_log: torch.Tensor, dt_bias: torch.Tensor, conv: torch.Tensor, key_heads: int, eps: float) -> bool:
     """Whether :func:`gdn_mixer` takes these arguments: head dims 128, four taps, plain contiguous tensors of the
-    dtypes the target keeps, at least one token, and no gradient asked for."""
+    dtypes the target keeps, at least one token, and nothing that autograd follows."""
     if not _residual(hidden):
         return False
     device = hidden.device
@@ -252,6 +259,7 @@ def gdn_mixer_fits(hidden: torch.Tensor, history: torch.Tensor, state: torch.Ten
             and _as(conv, b16, (width, 1, 4), device) and _as(norm, f32, (128,), device)
             and _as(input_norm, f32, (h,), device) and _as(post_norm, f32, (h,), device)
             and _as(a_log, f32, (hv,), device) and _as(dt_bias, f32, (hv,), device)
+            and not _tracked(hidden, history, state, conv, norm, input_norm, post_norm, a_log, dt_bias)
             and _matrix(in_proj, width + 128 * hv + 2 * hv, h, device) and _matrix(out_proj, h, 128 * hv, device))
 
 
@@ -259,7 +267,7 @@ def gdn_commit(state: torch.Tensor, keys: torch.Tensor, u: torch.Tensor, cum: to
                window: torch.Tensor, first: int) -> Optional[tuple]:
     """``(recurrent state, conv history)`` after the first ``accepted`` tokens of one chunk of :func:`gdn_mixer`
     (``layers.state_after`` and the window's columns ``[first, first + 3)``) in one launch; ``None`` when the tensors
-    are not laid out as that call leaves them."""
+    are not laid out as that call leaves them, or autograd follows them."""
     if _plain(state):
         done = _lib.host().commit(state, keys, u, cum, accepted, window, first)
         if done is not None:
@@ -271,7 +279,7 @@ def gdn_commit(state: torch.Tensor, keys: torch.Tensor, u: torch.Tensor, cum: to
             or any(t.dtype != torch.float32 or t.device != device for t in (keys, u, cum))
             or keys.stride()[2:] != (128, 1) or u.stride() != keys.stride() or cum.stride(2) != 1
             or window.dtype != torch.bfloat16 or window.ndim != 3 or window.shape[0] != 1 or window.device != device
-            or not window.is_contiguous() or first + 3 > window.shape[2]):
+            or not window.is_contiguous() or first + 3 > window.shape[2] or _tracked(state, keys, u, cum, window)):
         return None
     out = torch.empty_like(state)
     history = torch.empty((1, window.shape[1], 3), dtype=window.dtype, device=device)
@@ -286,7 +294,7 @@ def attention_mixer_fits(hidden: torch.Tensor, keys: torch.Tensor, values: torch
                          q_norm: torch.Tensor, k_norm: torch.Tensor, inv_freq: torch.Tensor, heads: int,
                          kv_heads: int, head_dim: int, eps: float) -> bool:
     """Whether :func:`attention_mixer` takes these arguments: head dim 128 or 256, plain contiguous tensors of the
-    dtypes the target keeps, room in the cache, and no gradient asked for."""
+    dtypes the target keeps, room in the cache, and nothing that autograd follows."""
     if not _residual(hidden) or head_dim not in (128, 256) or keys.ndim != 4 or keys.shape[2] > 1 << 24:
         return False
     device, (t, h) = hidden.device, hidden.shape
@@ -297,6 +305,7 @@ def attention_mixer_fits(hidden: torch.Tensor, keys: torch.Tensor, values: torch
             and _as(inv_freq, f32, (half,), device)
             and _as(input_norm, f32, (h,), device) and _as(post_norm, f32, (h,), device)
             and _as(q_norm, f32, (head_dim,), device) and _as(k_norm, f32, (head_dim,), device)
+            and not _tracked(hidden, keys, values, inv_freq, input_norm, post_norm, q_norm, k_norm)
             and _matrix(in_proj, 2 * (heads + kv_heads) * head_dim, h, device)
             and _matrix(out_proj, h, heads * head_dim, device))
 
@@ -499,6 +508,9 @@ def moe_w4a16_add(residual: torch.Tensor, hidden: torch.Tensor, gate_up: PackedW
     _require_device(router_weight)
     if router_weight.dtype != torch.bfloat16 or tuple(router_weight.shape) != (e, h):
         raise ValueError(f"router_weight must be bfloat16 [{e}, {h}]")
+    if _tracked(residual):
+        return residual + moe_w4a16(hidden, gate_up, down, top_k=top_k, router_weight=router_weight, shared=shared,
+                                    workspace=workspace).float()
     rw = router_weight.contiguous()
     logits = torch.empty((t, e), dtype=torch.float32, device=device)
     r = _routing_buffers(t, e, top_k, device)

@@ -175,3 +175,58 @@ def test_attention_over_an_infinite_key(pkg, device, kv_heads, group):
         else:
             assert torch.isfinite(general).all() and not torch.equal(general, want)
             assert metrics.compare(got.cpu() - x.cpu(), general.cpu() - x.cpu())["max_rel"] <= TOL
+
+
+@pytest.mark.parametrize("name", ["a_log", "dt_bias", "conv", "gdn_norm", "input_norm", "post_norm", "state"])
+def test_gdn_layer_keeps_gradients(pkg, device, name):
+    """Where a weight or the state asks for a gradient the PyTorch form runs, whose state and outputs carry it."""
+    c, _, model, state = _gdn_model(pkg, device, 4, 16, 8)
+    lw = model.w.layers[0]
+    leaf = state.recurrent[0] if name == "state" else getattr(lw, name)
+    leaf.requires_grad_()
+    x = torch.randn((8, c.hidden), generator=torch.Generator().manual_seed(3)).to(device)
+    args = model._gdn_args(lw)
+    assert not pkg.ops.gdn_mixer_fits(x, state.conv[0], state.recurrent[0], **args)
+    assert pkg.ops.gdn_mixer_plain(x, state.conv[0], state.recurrent[0], **args) is None
+    _, pending = model.layer(0, x, state)
+    assert pending.chunks[0].state.requires_grad == (name in ("a_log", "dt_bias", "conv", "state"))
+    model.commit(state, pkg.target.Pending(5, 8, [pending]), 3)
+    assert state.recurrent[0].requires_grad == (name in ("a_log", "dt_bias", "conv", "state"))
+    with torch.no_grad():
+        assert pkg.ops.gdn_mixer_plain(x, state.conv[0], state.recurrent[0].detach(), **args) is not None
+
+
+@pytest.mark.parametrize("name", ["q_norm", "k_norm", "input_norm", "post_norm"])
+def test_attention_layer_keeps_gradients(pkg, device, name):
+    c, model = _attention_model(pkg, device, 4, 2, 128, 32)
+    state, lw = model.synthetic_context(9, seed=4), model.w.layers[0]
+    getattr(lw, name).requires_grad_()
+    x = torch.randn((8, c.hidden), generator=torch.Generator().manual_seed(3)).to(device)
+    assert model._attention_kernels(x, lw, state.keys[0], state.values[0], 9) is None
+    model.layer(0, x, state)
+    assert state.keys[0].requires_grad == (name == "k_norm")
+
+
+@pytest.mark.parametrize("kind", ["linear_attention", "full_attention"])
+def test_layer_and_final_norm_keep_forward_tangents(pkg, device, kind):
+    """A forward-mode tangent of the residual goes through the residual adds and the final norm."""
+    import torch.autograd.forward_ad as fwd
+    c = pkg.target.small_config((kind,))
+    model = pkg.target.TargetModel(pkg.target.random_weights(c, seed=3, device=device), capacity=80)
+    x, v = (torch.randn((8, c.hidden), device=device) for _ in range(2))
+    with torch.no_grad(), fwd.dual_level():
+        dual = fwd.make_dual(x, v)
+        hidden, _ = model.layer(0, dual, model.synthetic_context(9, seed=4))
+        assert torch.equal(fwd.unpack_dual(hidden).tangent, v)
+        out = model.forward_hidden(dual, model.synthetic_context(9, seed=4), top1=False)
+        assert fwd.unpack_dual(out.hidden).tangent is not None
+
+
+def test_moe_residual_add_keeps_gradients(pkg, device):
+    layer = pkg.synthetic.moe_layer(4, hidden=512, inter=512, experts=16, seed=1)
+    x, banks = layer.hidden.to(device), (layer.gate_up.to(device), layer.down.to(device))
+    args = dict(top_k=4, router_weight=layer.router_weight.to(device))
+    residual = torch.randn((4, 512), device=device)
+    want = pkg.ops.moe_w4a16_add(residual, x, *banks, **args)
+    got = pkg.ops.moe_w4a16_add(residual.requires_grad_(), x, *banks, **args)
+    assert got.requires_grad and torch.equal(got, want)
