@@ -501,6 +501,8 @@ def moe_w4a16_add(residual: torch.Tensor, hidden: torch.Tensor, gate_up: PackedW
         if out is not None:
             return out
     device, flat, sgu, sdn, sgate = _moe_common(hidden, gate_up, down, shared)
+    if type(top_k) is not int:
+        raise ValueError("top_k must be an int")
     t, h = flat.shape
     e = gate_up.experts
     if not _as(residual, torch.float32, (t, h), device):

@@ -230,3 +230,12 @@ def test_moe_residual_add_keeps_gradients(pkg, device):
     want = pkg.ops.moe_w4a16_add(residual, x, *banks, **args)
     got = pkg.ops.moe_w4a16_add(residual.requires_grad_(), x, *banks, **args)
     assert got.requires_grad and torch.equal(got, want)
+
+
+@pytest.mark.parametrize("top_k", [True, 4.0])
+def test_moe_residual_add_refuses_other_counts(pkg, device, top_k):
+    """As moe_w4a16 does: an int, and no bool."""
+    layer = pkg.synthetic.moe_layer(4, hidden=512, inter=512, experts=16, seed=1)
+    with pytest.raises(ValueError, match="top_k must be an int"):
+        pkg.ops.moe_w4a16_add(torch.zeros((4, 512), device=device), layer.hidden.to(device), layer.gate_up.to(device),
+                              layer.down.to(device), top_k=top_k, router_weight=layer.router_weight.to(device))
