@@ -970,8 +970,8 @@ AttnLayout attn_layout(int64_t T, int64_t H, int64_t heads, int64_t kv, int64_t 
 }
 // The shapes the attention kernels take; row counts and cache offsets stay far inside 32 and 64 bits.
 bool attn_shape_ok(int64_t T, int64_t H, int64_t heads, int64_t kv, int64_t D) {
-  return T >= 0 && H > 0 && heads > 0 && kv > 0 && heads % kv == 0 && heads <= 1024 && (D == 128 || D == 256) &&
-         T * heads <= (int64_t(1) << 22);
+  return T >= 0 && T <= (int64_t(1) << 22) && H > 0 && heads > 0 && kv > 0 && heads % kv == 0 && heads <= 1024 &&
+         (D == 128 || D == 256) && T * heads <= (int64_t(1) << 22);
 }
 }  // namespace
 
@@ -993,7 +993,7 @@ int dflash_attention_mixer(const dflash_attention* a, const float* hidden, int64
       return fail(DFLASH_ERR_UNSUPPORTED, "attention: hidden_size must be a multiple of 512, at most 8192");
     if (a->rotary_dim <= 0 || a->rotary_dim > D || a->rotary_dim % (2 * (D / 64)))
       return fail(DFLASH_ERR_UNSUPPORTED, "attention: rotary_dim must be a multiple of head_dim / 32, at most head_dim");
-    if (position < 0 || capacity > (1 << 24) || position + T > capacity)
+    if (position < 0 || capacity > (1 << 24) || T > capacity || position > capacity - T)
       return fail(DFLASH_ERR_INVALID_ARGUMENT, "attention: block would exceed the KV cache capacity");
     const int64_t n_in = 2 * heads * D + 2 * kv * D;
     if (int r = check_w4(&a->in_proj, "attention in_proj", 1, n_in, H)) return r;

@@ -348,3 +348,32 @@ def test_build_goes_on_without_a_host_compiler(monkeypatch, tmp_path, capsys):
     assert not builder._finish_host(builder._start(["/bin/sh", "-c", "exit 1"]))
     assert builder._finish_host(builder._start(["/bin/sh", "-c", "exit 0"]))
     assert capsys.readouterr().err.count("is not built") == 2
+
+
+def _attention_args(pkg, tokens=1, position=0, capacity=64, heads=4, kv=2, d=128, hidden=512, layout=0, **over):
+    p = 1 << 20
+    desc = pkg._lib.AttentionDesc(
+        in_proj=_desc(pkg, rows=2 * (heads + kv) * d, cols=hidden, layout=layout), out_proj=_desc(pkg, rows=hidden, cols=heads * d, layout=layout),
+        input_norm=p, post_norm=p, q_norm=p, k_norm=p, inv_freq=p, hidden_size=hidden, heads=heads, kv_heads=kv, head_dim=d,
+        rotary_dim=d // 4, eps=1e-6)
+    for name, value in over.items():
+        setattr(desc, name, value)
+    v = ctypes.c_void_p(p)
+    return ctypes.byref(desc), v, tokens, position, v, v, capacity, v, v, v, 1 << 40, None
+
+
+@host_only
+@pytest.mark.parametrize("tokens,position,capacity", [
+    (1, (1 << 63) - 1, 64), (16, (1 << 63) - 16, 64), (2, 63, 64), (1, -1, 64), (65, 0, 64), (1, 0, 1 << 25), (1, 0, -(1 << 63))])
+def test_attention_block_outside_the_cache(pkg, tokens, position, capacity):
+    """Refused on the host, also where position + tokens leaves 64 bits."""
+    st, msg = _status(pkg, "dflash_attention_mixer", *_attention_args(pkg, tokens, position, capacity))
+    assert st == 1 and "capacity" in msg
+
+
+@host_only
+def test_attention_token_counts_past_64_bits(pkg):
+    """tokens * heads = 2^64 wraps to 0."""
+    st, msg = _status(pkg, "dflash_attention_mixer", *_attention_args(pkg, 1 << 62, 0, 64))
+    assert st == 2 and "2^22" in msg
+    assert pkg._lib.load().dflash_attention_workspace_bytes(1 << 62, 512, 4, 2, 128) == 0
