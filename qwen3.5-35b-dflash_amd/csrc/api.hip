@@ -917,15 +917,19 @@ int dflash_gdn_mixer(const dflash_gdn* g, const float* hidden, int64_t tokens, c
 
 int dflash_rms_norm(const float* hidden, int64_t tokens, int64_t hidden_size, const float* weight, float eps, float* out,
                     void* stream) {
-  if (tokens < 0 || tokens > (1 << 24)) return fail(DFLASH_ERR_UNSUPPORTED, "rms_norm: tokens must be in [0, 2^24]");
-  if (hidden_size <= 0 || hidden_size % 4 || hidden_size > dflash::kMaxNormWidth)
-    return fail(DFLASH_ERR_UNSUPPORTED, "rms_norm: hidden_size must be a multiple of 4, at most 8192");
-  if (tokens == 0) return DFLASH_OK;
-  if (!mixer_args_aligned({hidden, weight, out}))
-    return fail(DFLASH_ERR_INVALID_ARGUMENT, "rms_norm: NULL or misaligned pointer");
-  dflash::launch_norm_f32(hidden, weight, eps, static_cast<int>(tokens), static_cast<int>(hidden_size), out,
-                          static_cast<hipStream_t>(stream));
-  return launch_status("rms_norm");
+  try {
+    if (tokens < 0 || tokens > (1 << 24)) return fail(DFLASH_ERR_UNSUPPORTED, "rms_norm: tokens must be in [0, 2^24]");
+    if (hidden_size <= 0 || hidden_size % 4 || hidden_size > dflash::kMaxNormWidth)
+      return fail(DFLASH_ERR_UNSUPPORTED, "rms_norm: hidden_size must be a multiple of 4, at most 8192");
+    if (tokens == 0) return DFLASH_OK;
+    if (!mixer_args_aligned({hidden, weight, out}))
+      return fail(DFLASH_ERR_INVALID_ARGUMENT, "rms_norm: NULL or misaligned pointer");
+    dflash::launch_norm_f32(hidden, weight, eps, static_cast<int>(tokens), static_cast<int>(hidden_size), out,
+                            static_cast<hipStream_t>(stream));
+    return launch_status("rms_norm");
+  } catch (...) {
+    return fail(DFLASH_ERR_HIP, "unexpected host exception");
+  }
 }
 
 int dflash_gdn_commit(const float* state, const float* keys, const float* u, const float* cum, int64_t head_stride,

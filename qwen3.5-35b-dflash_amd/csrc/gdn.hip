@@ -433,7 +433,10 @@ void launch_add_norm(const float* hidden, const uint16_t* mixed, const float* w,
 }
 
 void launch_norm_f32(const float* hidden, const float* w, float eps, int T, int H, float* normed, hipStream_t stream) {
-  hipLaunchKernelGGL(add_norm_kernel<true>, dim3(T), dim3(512), 0, stream, hidden, nullptr, w, eps, H, nullptr, normed);
+  constexpr int kRows = 1 << 22;  // a launch stays below 2^32 work-items
+  for (int t = 0; t < T; t += kRows)
+    hipLaunchKernelGGL(add_norm_kernel<true>, dim3(min(kRows, T - t)), dim3(512), 0, stream, hidden + static_cast<int64_t>(t) * H,
+                       nullptr, w, eps, H, nullptr, normed + static_cast<int64_t>(t) * H);
 }
 
 void launch_gdn(const GdnParams& p, hipStream_t stream) {

@@ -187,3 +187,13 @@ def test_two_commits_of_one_block_share_nothing(pkg, device, tokens, accepted):
         commits.append(branch)
     assert len({t.untyped_storage().data_ptr() for b in commits for t in (b.conv[0], b.recurrent[0])}) == 6
     assert torch.equal(state.conv[0], before.conv[0]) and torch.equal(state.recurrent[0], before.recurrent[0])
+
+
+def test_rms_norm_of_more_rows_than_one_launch_holds(pkg, device):
+    """2^23 + 3 rows at 512 threads each are more than 2^32 work-items: three launches (4 columns, in place)."""
+    tokens = (1 << 23) + 3
+    x = torch.randn((tokens, 4), device=device)
+    w = torch.randn((4,), device=device)
+    want = x * (x.square().mean(-1, keepdim=True) + 1e-6).rsqrt() * (w + 1)
+    pkg._lib.call("dflash_rms_norm", pkg.ops._ptr(x), tokens, 4, pkg.ops._ptr(w), 1e-6, pkg.ops._ptr(x), pkg.ops._stream(device))
+    torch.testing.assert_close(x, want, rtol=1e-6, atol=1e-6)     # a few fp32 roundings each
