@@ -689,7 +689,6 @@ size_t dflash_qlinear_workspace_bytes(int64_t m, int64_t k, int64_t group_size) 
 }
 
 namespace {
-// Both qlinear entry points: y is bf16 [m][N], or fp32 when y_f32.
 // 16-row blocks (w4_small.hip): the one-round-trip kernel up to N = 8192, its streaming form
 // (x kept in registers, persistent workgroups) up to N = 32768, the staging verify kernel
 // above (measured per projection: N = 8192 6.5 against 7.6 us streaming; N = 9216 7.5 against
@@ -697,32 +696,77 @@ namespace {
 constexpr int64_t kSmallLinearMaxN = 8192;
 constexpr int64_t kSmallStreamMinN = 8193, kSmallStreamMaxN = 32768;
 
+int check_qlinear(int64_t m, const dflash_w4* weight) {
+  if (!weight) return fail(DFLASH_ERR_INVALID_ARGUMENT, "weight descriptor is NULL");
+  if (m < 0) return fail(DFLASH_ERR_INVALID_ARGUMENT, "m must be >= 0");
+  if (m > (1 << 24)) return fail(DFLASH_ERR_UNSUPPORTED, "m above 2^24 is not supported");
+  const int64_t N = weight->rows, K = weight->cols;
+  if (int r = check_w4(weight, "weight", 1, N, K)) return r;
+  if (N <= 0 || N % 32) return fail(DFLASH_ERR_UNSUPPORTED, "qlinear needs N % 32 == 0");
+  if (K <= 0 || K % 512) return fail(DFLASH_ERR_UNSUPPORTED, "qlinear needs K % 512 == 0");
+  return DFLASH_OK;
+}
+
+// The kernel that takes m >= 1 rows of a matrix check_qlinear passed, or why none does; launches nothing.
+enum class LinearPath { kSmall, kSmallStream, kVerify, kLinear };
+int qlinear_path(int64_t m, const dflash_w4* weight, LinearPath* path, dflash::VerifyParams* vl, int64_t* vrows) {
+  const int64_t N = weight->rows, K = weight->cols;
+  const int im = static_cast<int>(m), in = static_cast<int>(N), ik = static_cast<int>(K),
+            ig = static_cast<int>(weight->group_size);
+  // narrow projections of a short block: the one-round-trip kernel (operands straight into
+  // MFMA fragments, one workgroup per 16 columns); wider ones stage x once per workgroup
+  if (N >= kSmallStreamMinN && N <= kSmallStreamMaxN && dflash::small_linear_stream_fits(im, in, ik, ig)) {
+    *path = LinearPath::kSmallStream;
+    return DFLASH_OK;
+  }
+  if (N <= kSmallLinearMaxN && dflash::small_linear_fits(im, in, ik, ig)) {
+    *path = LinearPath::kSmall;
+    return DFLASH_OK;
+  }
+  // the verify kernel for the wide outputs of up to 32 rows, else w4_linear.  The verify kernel stages at most 16 rows of
+  // K = 4096; 17..32 rows run as two launches of it
+  *vrows = K == 4096 && m > 16 && m <= 32 ? 16 : m;
+  if ((ig == 128 || ig == 256) &&
+      dflash::verify_layout(dflash::kModeLinear, static_cast<int>(*vrows), ik, in, 1, 1, 0, 0, vl)) {
+    *path = LinearPath::kVerify;
+    return DFLASH_OK;
+  }
+  // tiled banks are taken in the shapes the contract names (group 128, K of 512, 1024 or 2048, N a multiple of
+  // 32 times the row groups above 32 rows), not in all that the kernel could read
+  if (weight->layout == DFLASH_LAYOUT_TILED && !w4_path_reads_tiled(dflash::kModeLinear, in, ik, ig, GemmPath::kStream))
+    return tiled_unsupported("qlinear");
+  if (!dflash::w4_linear_fits(m, N, K)) return fail(DFLASH_ERR_UNSUPPORTED, "qlinear: K must stay below 2^25");
+  *path = LinearPath::kLinear;
+  return DFLASH_OK;
+}
+
+// Whether a mixer's projection of T >= 1 rows has a kernel, before the mixer launches or writes anything.
+int check_projection(int64_t T, const dflash_w4* weight) {
+  LinearPath path;
+  dflash::VerifyParams vl{};
+  int64_t vrows;
+  if (int r = check_qlinear(T, weight)) return r;
+  return qlinear_path(T, weight, &path, &vl, &vrows);
+}
+
+// Both qlinear entry points: y is bf16 [m][N], or fp32 when y_f32.
 int qlinear_impl(const void* x, int64_t m, const dflash_w4* weight, void* y, bool y_f32, void* workspace,
                  size_t workspace_bytes, void* stream) {
   try {
-    if (!weight) return fail(DFLASH_ERR_INVALID_ARGUMENT, "weight descriptor is NULL");
-    if (m < 0) return fail(DFLASH_ERR_INVALID_ARGUMENT, "m must be >= 0");
-    if (m > (1 << 24)) return fail(DFLASH_ERR_UNSUPPORTED, "m above 2^24 is not supported");
-    const int64_t N = weight->rows, K = weight->cols;
-    if (int r = check_w4(weight, "weight", 1, N, K)) return r;
-    if (N <= 0 || N % 32) return fail(DFLASH_ERR_UNSUPPORTED, "qlinear needs N % 32 == 0");
-    if (K <= 0 || K % 512) return fail(DFLASH_ERR_UNSUPPORTED, "qlinear needs K % 512 == 0");
+    if (int r = check_qlinear(m, weight)) return r;
     if (m == 0) return DFLASH_OK;
+    const int64_t N = weight->rows, K = weight->cols;
     if (!x || !y || !aligned16(x) || !aligned16(y)) return fail(DFLASH_ERR_INVALID_ARGUMENT, "x/y NULL or not 16-byte aligned");
     const size_t need = dflash_qlinear_workspace_bytes(m, K, weight->group_size);
     if (!workspace || workspace_bytes < need || !aligned16(workspace))
       return fail(DFLASH_ERR_WORKSPACE, "qlinear workspace needs " + std::to_string(need) + " bytes");
     hipStream_t st = static_cast<hipStream_t>(stream);
     const bool tiled = weight->layout == DFLASH_LAYOUT_TILED;
-    // narrow projections of a short block: the one-round-trip kernel (operands straight into
-    // MFMA fragments, one workgroup per 16 columns); wider ones stage x once per workgroup
-    const bool stream_form =
-        N >= kSmallStreamMinN && N <= kSmallStreamMaxN && dflash::small_linear_stream_fits(static_cast<int>(m), static_cast<int>(N),
-                                                                   static_cast<int>(K),
-                                                                   static_cast<int>(weight->group_size));
-    if (stream_form || (N <= kSmallLinearMaxN &&
-                        dflash::small_linear_fits(static_cast<int>(m), static_cast<int>(N), static_cast<int>(K),
-                                                  static_cast<int>(weight->group_size)))) {
+    LinearPath path;
+    dflash::VerifyParams vl{};
+    int64_t vrows = m;
+    if (int r = qlinear_path(m, weight, &path, &vl, &vrows)) return r;
+    if (path == LinearPath::kSmall || path == LinearPath::kSmallStream) {
       dflash::SmallLinearParams sp{};
       sp.x = static_cast<const uint16_t*>(x);
       sp.w = static_cast<const uint8_t*>(weight->packed);
@@ -735,24 +779,11 @@ int qlinear_impl(const void* x, int64_t m, const dflash_w4* weight, void* y, boo
       sp.tiled = tiled ? 1 : 0;
       sp.scale_f32 = weight->scale_dtype == DFLASH_DTYPE_F32 ? 1 : 0;
       sp.y_f32 = y_f32 ? 1 : 0;
-      if (stream_form) dflash::launch_w4_small_stream(sp, cu_count(), st);
+      if (path == LinearPath::kSmallStream) dflash::launch_w4_small_stream(sp, cu_count(), st);
       else dflash::launch_w4_small(sp, st);
       return launch_status("qlinear");
     }
-    // the verify kernel for the wide outputs of up to 32 rows, else w4_linear
-    dflash::VerifyParams vl{};
-    // the verify kernel stages at most 16 rows of K = 4096; 17..32 rows run as two launches of it
-    const int64_t vrows = K == 4096 && m > 16 && m <= 32 ? 16 : m;
-    const bool verify = (weight->group_size == 128 || weight->group_size == 256) &&
-                        dflash::verify_layout(dflash::kModeLinear, static_cast<int>(vrows), static_cast<int>(K),
-                                              static_cast<int>(N), 1, 1, 0, 0, &vl);
-    // tiled banks are taken in the shapes the contract names (group 128, K of 512, 1024 or 2048, N a multiple of
-    // 32 times the row groups above 32 rows), not in all that the kernel could read
-    if (tiled && !verify &&
-        !w4_path_reads_tiled(dflash::kModeLinear, static_cast<int>(N), static_cast<int>(K),
-                             static_cast<int>(weight->group_size), GemmPath::kStream))
-      return tiled_unsupported("qlinear");
-    if (verify) {
+    if (path == LinearPath::kVerify) {
       dflash::W4StreamParams p{};
       p.w = static_cast<const uint8_t*>(weight->packed);
       p.s = weight->scales;
@@ -776,7 +807,6 @@ int qlinear_impl(const void* x, int64_t m, const dflash_w4* weight, void* y, boo
       }
       return DFLASH_OK;
     }
-    if (!dflash::w4_linear_fits(m, N, K)) return fail(DFLASH_ERR_UNSUPPORTED, "qlinear: K must stay below 2^25");
     const size_t rows = (static_cast<size_t>(m) + 31) / 32 * 32;
     Carver c;
     dflash::LinearParams lp{};
@@ -861,6 +891,8 @@ int dflash_gdn_mixer(const dflash_gdn* g, const float* hidden, int64_t tokens, c
     if (int r = check_w4(&g->in_proj, "gdn in_proj", 1, n_in, H)) return r;
     if (int r = check_w4(&g->out_proj, "gdn out_proj", 1, H, vw)) return r;
     if (T == 0) return DFLASH_OK;
+    if (int r = check_projection(T, &g->in_proj)) return r;
+    if (int r = check_projection(T, &g->out_proj)) return r;
     if (!mixer_args_aligned({g->input_norm, g->post_norm, g->norm, g->conv, hidden, history, state, mid, normed, window,
                              tail, states, keys, u, cum, core}) || !g->a_log || !g->dt_bias)
       return fail(DFLASH_ERR_INVALID_ARGUMENT, "gdn: NULL or misaligned pointer");
@@ -1003,6 +1035,8 @@ int dflash_attention_mixer(const dflash_attention* a, const float* hidden, int64
     if (int r = check_w4(&a->in_proj, "attention in_proj", 1, n_in, H)) return r;
     if (int r = check_w4(&a->out_proj, "attention out_proj", 1, H, heads * D)) return r;
     if (T == 0) return DFLASH_OK;
+    if (int r = check_projection(T, &a->in_proj)) return r;
+    if (int r = check_projection(T, &a->out_proj)) return r;
     if (!mixer_args_aligned({a->input_norm, a->post_norm, a->q_norm, a->k_norm, hidden, keys, values, mid, normed}) ||
         !a->inv_freq)
       return fail(DFLASH_ERR_INVALID_ARGUMENT, "attention: NULL or misaligned pointer");

@@ -377,3 +377,20 @@ def test_attention_token_counts_past_64_bits(pkg):
     st, msg = _status(pkg, "dflash_attention_mixer", *_attention_args(pkg, 1 << 62, 0, 64))
     assert st == 2 and "2^22" in msg
     assert pkg._lib.load().dflash_attention_workspace_bytes(1 << 62, 512, 4, 2, 128) == 0
+
+
+@host_only
+def test_mixers_refuse_a_projection_without_a_kernel(pkg):
+    """Tiled K = 4096 above 32 rows, and N that is no multiple of 32: status 2 from the host, before the norm, the cache
+    rows or anything else is launched (which would report the missing device)."""
+    st, msg = _status(pkg, "dflash_attention_mixer", *_attention_args(pkg, 33, 0, 64, heads=16, d=256, layout=1))
+    assert st == 2 and "tiled" in msg
+    st, msg = _status(pkg, "dflash_attention_mixer", *_attention_args(pkg, 1, 0, 64, heads=6, kv=3, d=128))
+    assert st == 2 and "K % 512" in msg
+    v = ctypes.c_void_p(1 << 20)
+    for tokens, hk, hv, layout, why in ((33, 16, 32, 1, "tiled"), (1, 4, 4, 0, "N % 32"), (1, 4, 16, 0, None)):
+        desc = pkg._lib.GdnDesc(
+            in_proj=_desc(pkg, rows=256 * hk + 258 * hv, cols=512, layout=layout), out_proj=_desc(pkg, rows=512, cols=128 * hv, layout=layout),
+            input_norm=v, post_norm=v, norm=v, a_log=v, dt_bias=v, conv=v, hidden_size=512, key_heads=hk, value_heads=hv, eps=1e-6)
+        st, msg = _status(pkg, "dflash_gdn_mixer", ctypes.byref(desc), v, tokens, v, v, v, v, v, v, v, v, v, v, v, v, 16, None)
+        assert (st, why in msg) == (2, True) if why else (st, "workspace" in msg) == (3, True)
