@@ -190,7 +190,7 @@ def host():
             loader.exec_module(module)
             if module.TORCH != torch.__version__:
                 raise ImportError(f"built for torch {module.TORCH}, not {torch.__version__}")
-            module.bind(PackedW4, SharedExpert, lambda name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value)
+            module.bind(PackedW4, SharedExpert, check, lambda name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value)
             _HOST = module
         except (ImportError, AttributeError) as error:
             warnings.warn(f"{HOST_PATH.name} is not used ({error}); calls take their Python form, build.py builds it",

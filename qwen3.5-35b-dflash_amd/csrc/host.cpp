@@ -5,8 +5,9 @@
 // allocations); a 16-token GDN layer 89 us of device time behind 156 us of it.  Every function here takes the arguments
 // of its namesake in ops.py, does what that does when they are plain (exact torch.Tensor and bank types, contiguous, on
 // one ROCm device, no dispatch or function mode active) and returns None otherwise, before anything is launched; ops.py
-// then takes its own path, which decides and reports as it always did.  No state but the entry points' addresses and
-// the two bank types, set once by bind().  The GIL is released while an entry enqueues.
+// then takes its own path, which decides and reports as it always did.  A call that its entry refuses raises what ops.py
+// would (_lib.check).  No state but the entry points' addresses, the two bank types and that function, set once by
+// bind().  The GIL is released while an entry enqueues.
 #include <ATen/ATen.h>
 #include <ATen/PythonTorchFunctionTLS.h>
 #include <ATen/TensorSubclassLikeUtils.h>
@@ -21,6 +22,7 @@ namespace {
 
 PyTypeObject* g_packed_type = nullptr;
 PyTypeObject* g_shared_type = nullptr;
+PyObject* g_check = nullptr;
 
 struct Entries {
   decltype(&dflash_qlinear_workspace_bytes) qlinear_workspace_bytes;
@@ -36,6 +38,14 @@ struct Entries {
   decltype(&dflash_attention_workspace_bytes) attention_workspace_bytes;
   decltype(&dflash_attention_mixer) attention;
 } g_entry;
+
+// _lib.check of a nonzero status: raises DflashError with the library's message
+PyObject* refused(const char* entry, int status) {
+  PyObject* r = PyObject_CallFunction(g_check, "si", entry, status);
+  if (r) PyErr_SetString(PyExc_SystemError, "a refused call was not reported");
+  Py_XDECREF(r);
+  return nullptr;
+}
 
 bool plain_state() { return !c10::impl::dispatch_mode_enabled() && !at::impl::torch_function_mode_enabled(); }
 
@@ -144,7 +154,7 @@ PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (f32) status = g_entry.qlinear_f32(x->data_ptr(), m, &w, static_cast<float*>(y.data_ptr()), ws.data_ptr(), ws.numel(), st);
   else status = g_entry.qlinear(x->data_ptr(), m, &w, y.data_ptr(), ws.data_ptr(), ws.numel(), st);
   Py_END_ALLOW_THREADS
-  if (status) Py_RETURN_NONE;
+  if (status) return refused(f32 ? "dflash_qlinear_w4a16_f32" : "dflash_qlinear_w4a16", status);
   return THPVariable_Wrap(std::move(y));
   END_HANDLE_TH_ERRORS
 }
@@ -207,7 +217,7 @@ PyObject* moe(PyObject*, PyObject* const* a, Py_ssize_t n) {
                          reinterpret_cast<float*>(logits), ids, reinterpret_cast<float*>(wts), perm, inv, offsets,
                          ws.data_ptr(), ws.numel(), st);
   Py_END_ALLOW_THREADS
-  if (status) Py_RETURN_NONE;
+  if (status) return refused(residual ? "dflash_moe_w4a16_residual" : "dflash_moe_w4a16", status);
   return THPVariable_Wrap(std::move(out));
   END_HANDLE_TH_ERRORS
 }
@@ -248,8 +258,8 @@ PyObject* gdn(PyObject*, PyObject* const* a, Py_ssize_t n) {
   dflash_gdn g{};
   if (!history || !state || !input_norm || !post_norm || !norm || !dt_bias || !conv ||
       tracked(*history) || tracked(*state) || tracked(*input_norm) || tracked(*post_norm) || tracked(*norm) ||
-      tracked(*dt_bias) || tracked(*conv) || tracked(*a_log) || !exactly(a[8], at::kFloat, {hv}, device) || !matrix(a[3], width + 128 * hv + 2 * hv, h, device, &g.in_proj) ||
-      !matrix(a[4], h, 128 * hv, device, &g.out_proj))
+      tracked(*dt_bias) || tracked(*conv) || tracked(*a_log) || !exactly(a[8], at::kFloat, {hv}, device) ||
+      !matrix(a[3], width + 128 * hv + 2 * hv, h, device, &g.in_proj) || !matrix(a[4], h, 128 * hv, device, &g.out_proj))
     Py_RETURN_NONE;
   g.input_norm = static_cast<const float*>(input_norm->data_ptr());
   g.post_norm = static_cast<const float*>(post_norm->data_ptr());
@@ -275,7 +285,7 @@ PyObject* gdn(PyObject*, PyObject* const* a, Py_ssize_t n) {
                        static_cast<const float*>(state->data_ptr()), f(0), o[1].data_ptr(), o[2].data_ptr(), o[3].data_ptr(), f(4),
                        f(5), f(6), f(7), f(8), ws.data_ptr(), ws.numel(), st);
   Py_END_ALLOW_THREADS
-  if (status) Py_RETURN_NONE;
+  if (status) return refused("dflash_gdn_mixer", status);
   PyObject* r = PyTuple_New(9);
   for (int i = 0; r && i < 9; ++i) PyTuple_SET_ITEM(r, i, THPVariable_Wrap(std::move(o[i])));
   return r;
@@ -297,7 +307,7 @@ PyObject* rms_norm(PyObject*, PyObject* const* a, Py_ssize_t n) {
                             static_cast<const float*>(w->data_ptr()), static_cast<float>(PyFloat_AS_DOUBLE(a[2])),
                             static_cast<float*>(out.data_ptr()), st);
   Py_END_ALLOW_THREADS
-  if (status) Py_RETURN_NONE;
+  if (status) return refused("dflash_rms_norm", status);
   return THPVariable_Wrap(std::move(out));
   END_HANDLE_TH_ERRORS
 }
@@ -334,8 +344,8 @@ PyObject* attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
   dflash_attention g{};
   if (!exactly(a[1], at::kBFloat16, cache, device) || !values || !input_norm || !post_norm || !q_norm || !k_norm ||
       tracked(*keys) || tracked(*values) || tracked(*input_norm) || tracked(*post_norm) || tracked(*q_norm) ||
-      tracked(*k_norm) || tracked(*inv_freq) || !exactly(a[10], at::kFloat, {half}, device) || !matrix(a[4], 2 * (heads + kv) * d, h, device, &g.in_proj) ||
-      !matrix(a[5], h, heads * d, device, &g.out_proj))
+      tracked(*k_norm) || tracked(*inv_freq) || !exactly(a[10], at::kFloat, {half}, device) ||
+      !matrix(a[4], 2 * (heads + kv) * d, h, device, &g.in_proj) || !matrix(a[5], h, heads * d, device, &g.out_proj))
     Py_RETURN_NONE;
   g.input_norm = static_cast<const float*>(input_norm->data_ptr());
   g.post_norm = static_cast<const float*>(post_norm->data_ptr());
@@ -356,7 +366,7 @@ PyObject* attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
   status = g_entry.attention(&g, static_cast<const float*>(x->data_ptr()), t, position, keys->data_ptr(), values->data_ptr(),
                              keys->size(2), static_cast<float*>(mid.data_ptr()), normed.data_ptr(), ws.data_ptr(), ws.numel(), st);
   Py_END_ALLOW_THREADS
-  if (status) Py_RETURN_NONE;
+  if (status) return refused("dflash_attention_mixer", status);
   PyObject* r = PyTuple_New(2);
   if (r) {
     PyTuple_SET_ITEM(r, 0, THPVariable_Wrap(std::move(mid)));
@@ -377,8 +387,8 @@ PyObject* commit(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const int64_t j = PyLong_AsLong(a[4]), first = PyLong_AsLong(a[6]), hv = state->size(1);
   const at::Device device = state->device();
   const auto f32 = [&](const at::Tensor* t) { return t->scalar_type() == at::kFloat && t->device() == device; };
-  if (j < 1 || j > 16 || first < 0 || !exactly(a[0], at::kFloat, {1, hv, 128, 128}, device) || keys->dim() != 4 ||
-      keys->size(0) != 1 || keys->size(1) != hv || keys->size(2) < j || keys->size(3) != 128 || u->sizes() != keys->sizes() ||
+  if (j < 1 || j > 16 || first < 0 || first > 1 << 24 || hv > 1024 ||
+      !exactly(a[0], at::kFloat, {1, hv, 128, 128}, device) || keys->dim() != 4 || keys->size(0) != 1 || keys->size(1) != hv || keys->size(2) < j || keys->size(3) != 128 || u->sizes() != keys->sizes() ||
       cum->sizes() != keys->sizes().slice(0, 3) || !f32(keys) || !f32(u) || !f32(cum) || keys->stride(2) != 128 ||
       keys->stride(3) != 1 || u->strides() != keys->strides() || cum->stride(2) != 1 ||
       window->scalar_type() != at::kBFloat16 || window->dim() != 3 || window->size(0) != 1 || window->device() != device ||
@@ -396,7 +406,7 @@ PyObject* commit(PyObject*, PyObject* const* a, Py_ssize_t n) {
                           static_cast<float*>(out.data_ptr()), window->data_ptr(), window->size(2), first, window->size(1),
                           history.data_ptr(), st);
   Py_END_ALLOW_THREADS
-  if (status) Py_RETURN_NONE;
+  if (status) return refused("dflash_gdn_commit", status);
   PyObject* r = PyTuple_New(2);
   if (r) {
     PyTuple_SET_ITEM(r, 0, THPVariable_Wrap(std::move(out)));
@@ -406,10 +416,10 @@ PyObject* commit(PyObject*, PyObject* const* a, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
-// bind(PackedW4, SharedExpert, address of an entry by name)
+// bind(PackedW4, SharedExpert, _lib.check, address of an entry by name)
 PyObject* bind(PyObject*, PyObject* args) {
-  PyObject *packed, *shared, *find;
-  if (!PyArg_ParseTuple(args, "O!O!O", &PyType_Type, &packed, &PyType_Type, &shared, &find)) return nullptr;
+  PyObject *packed, *shared, *check, *find;
+  if (!PyArg_ParseTuple(args, "O!O!OO", &PyType_Type, &packed, &PyType_Type, &shared, &check, &find)) return nullptr;
   bool ok = true;
   const auto get = [&](const char* name, auto& fn) {
     PyObject* v = ok ? PyObject_CallFunction(find, "s", name) : nullptr;
@@ -436,6 +446,8 @@ PyObject* bind(PyObject*, PyObject* args) {
   }
   Py_INCREF(packed);
   Py_INCREF(shared);
+  Py_INCREF(check);
+  g_check = check;
   g_packed_type = reinterpret_cast<PyTypeObject*>(packed);
   g_shared_type = reinterpret_cast<PyTypeObject*>(shared);
   Py_RETURN_NONE;

@@ -273,7 +273,8 @@ def gdn_commit(state: torch.Tensor, keys: torch.Tensor, u: torch.Tensor, cum: to
         if done is not None:
             return done
     hv, device = state.shape[1], state.device
-    if (device.type != "cuda" or not 1 <= accepted <= 16 or not _as(state, torch.float32, (1, hv, 128, 128), device)
+    if (device.type != "cuda" or not 1 <= accepted <= 16 or hv > 1024 or not 0 <= first <= 1 << 24
+            or not _as(state, torch.float32, (1, hv, 128, 128), device)
             or keys.shape[:2] != (1, hv) or keys.shape[2] < accepted or keys.shape[3] != 128 or u.shape != keys.shape
             or cum.shape != keys.shape[:3]
             or any(t.dtype != torch.float32 or t.device != device for t in (keys, u, cum))

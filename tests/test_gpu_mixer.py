@@ -239,3 +239,18 @@ def test_moe_residual_add_refuses_other_counts(pkg, device, top_k):
     with pytest.raises(ValueError, match="top_k must be an int"):
         pkg.ops.moe_w4a16_add(torch.zeros((4, 512), device=device), layer.hidden.to(device), layer.gate_up.to(device),
                               layer.down.to(device), top_k=top_k, router_weight=layer.router_weight.to(device))
+
+
+@pytest.mark.parametrize("kind", ["linear_attention", "full_attention"])
+def test_a_refused_projection_leaves_the_cache_as_it_was(pkg, device, kind, monkeypatch):
+    """Tiled K = 4096 above 32 rows has no kernel: the layer is refused, once, before anything is launched or written."""
+    base = pkg.target.small_config((kind,))
+    c = type(base)(**{**vars(base), "heads": 16, "head_dim": 256, "linear_key_heads": 16, "linear_value_heads": 32})
+    model = pkg.target.TargetModel(pkg.target.random_weights(c, seed=3, device=device, layout="tiled"), capacity=80)
+    state = model.synthetic_context(9, seed=4)
+    before = state.clone()
+    monkeypatch.setattr(pkg._lib, "call", None)          # the Python form is not tried
+    with pytest.raises(pkg._lib.DflashError, match="tiled"):
+        model.layer(0, torch.randn((40, c.hidden), device=device), state)
+    for a, b in zip(state.keys + state.values, before.keys + before.values):
+        assert (a is None and b is None) or torch.equal(a, b)
