@@ -388,7 +388,8 @@ PyObject* commit(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const at::Device device = state->device();
   const auto f32 = [&](const at::Tensor* t) { return t->scalar_type() == at::kFloat && t->device() == device; };
   if (j < 1 || j > 16 || first < 0 || first > 1 << 24 || hv > 1024 ||
-      !exactly(a[0], at::kFloat, {1, hv, 128, 128}, device) || keys->dim() != 4 || keys->size(0) != 1 || keys->size(1) != hv || keys->size(2) < j || keys->size(3) != 128 || u->sizes() != keys->sizes() ||
+      !exactly(a[0], at::kFloat, {1, hv, 128, 128}, device) || keys->dim() != 4 || keys->size(0) != 1 ||
+      keys->size(1) != hv || keys->size(2) < j || keys->size(3) != 128 || u->sizes() != keys->sizes() ||
       cum->sizes() != keys->sizes().slice(0, 3) || !f32(keys) || !f32(u) || !f32(cum) || keys->stride(2) != 128 ||
       keys->stride(3) != 1 || u->strides() != keys->strides() || cum->stride(2) != 1 ||
       window->scalar_type() != at::kBFloat16 || window->dim() != 3 || window->size(0) != 1 || window->device() != device ||

@@ -789,22 +789,6 @@ __global__ __launch_bounds__(512) void table_prep_kernel(TableParams p) {
   }
 }
 
-// Four columns of the layer's output: bf16, or that bf16 value added to the residual in fp32.
-__device__ __forceinline__ void store_combined(const CombineOut& out, int64_t at, float4 v) {
-  const uint32_t lo = f32_to_bf16(v.x) | (static_cast<uint32_t>(f32_to_bf16(v.y)) << 16);
-  const uint32_t hi = f32_to_bf16(v.z) | (static_cast<uint32_t>(f32_to_bf16(v.w)) << 16);
-  if (out.sum == nullptr) {
-    *reinterpret_cast<uint2*>(out.bf16 + at) = make_uint2(lo, hi);
-    return;
-  }
-  float4 r = *reinterpret_cast<const float4*>(out.residual + at);
-  r.x += __uint_as_float(lo << 16);
-  r.y += __uint_as_float(lo & 0xFFFF0000u);
-  r.z += __uint_as_float(hi << 16);
-  r.w += __uint_as_float(hi & 0xFFFF0000u);
-  *reinterpret_cast<float4*>(out.sum + at) = r;
-}
-
 // N columns of the layer's output from `at`: bf16, or (kSum) those bf16 values added to the residual in fp32.
 template <bool kSum, int N>
 __device__ __forceinline__ void store_combined(const CombineOut& out, int64_t at, const float (&v)[N]) {
@@ -828,6 +812,17 @@ __device__ __forceinline__ void store_combined(const CombineOut& out, int64_t at
   }
 }
 
+// ---------------------------------------------------------------------------
+// Combine: the layer's row t = sum_slot y[inv[t*k+slot]] (+ y[T*k + t] for the shared
+// expert), fp32 in slot order, one bf16 rounding, left as bf16 or (kSum) added to the residual.
+// y rows are fp32, or bf16 (the prefill tile path, already weighted).  When wts is given the rows
+// are unweighted expert outputs and each is scaled first: by wts[t*k+slot]
+// (the routing weight) or gate[t] (the shared-expert sigmoid) -- the same fp32
+// product the expert epilogues otherwise apply.  grid = (T, H / 512),
+// block = 64: a lane owns 8 columns; the rows are read kBatch at a time, all
+// loads of a batch in flight together, and added in slot order.  fp32 rows come
+// from verify blocks (top-k + the shared expert: 9 rows at top-8), read in one
+// batch of 16; the prefill's bf16 rows stream in batches of 8.
 template <typename YT, bool kSum>
 __global__ __launch_bounds__(64) void combine_kernel(const YT* __restrict__ y, const int32_t* __restrict__ inv, int T,
                                                      int k, int H, int has_shared, const float* __restrict__ wts,

@@ -34,7 +34,6 @@
 namespace dflash {
 namespace {
 
-constexpr float kOffset = 24.0f;
 constexpr uint32_t kMinus24Pair = 0xC1C0C1C0u;  // bf16 pair (-24, -24)
 
 // 8 signed nibbles -> 4 bf16 pairs (k0,k4) (k1,k5) (k2,k6) (k3,k7) holding 24 + q: the nibble with its sign bit
@@ -513,8 +512,7 @@ bool w4_linear_fits(int64_t M, int64_t N, int64_t K) {
 }
 
 void launch_w4_linear(const LinearParams& p, int cus, hipStream_t stream) {
-  const int64_t waves = static_cast<int64_t>((p.M + 31) / 32) * (p.K / 128);
-  hipLaunchKernelGGL(w4_linear_prep_kernel, dim3(static_cast<unsigned>((waves + 3) / 4)), dim3(256), 0, stream, p);
+  launch_prep(p, stream);
   const int64_t tiles = static_cast<int64_t>((p.M + 32 * kSub - 1) / (32 * kSub)) * ((p.N + 255) / 256);
   if (8 * tiles >= 5 * cus) {
     const dim3 grid(static_cast<unsigned>((tiles + 7) / 8 * 8)), block(256);
