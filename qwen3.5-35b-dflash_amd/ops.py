@@ -122,16 +122,18 @@ def to_tiled(w: PackedW4) -> PackedW4:
 
 
 def _plain(x) -> bool:
-    """Whether a call on ``x`` is first offered to the native form (``csrc/host.cpp``), which takes it or returns None."""
-    return type(x) is torch.Tensor and x.is_cuda and _lib.host() is not None
+    """Whether a call on ``x`` is first offered to the native form (``csrc/host.cpp``, where there is one), which takes it
+    or returns None."""
+    return type(x) is torch.Tensor and x.is_cuda
 
 
 def qlinear(x: torch.Tensor, weight: PackedW4, *, workspace: Optional[torch.Tensor] = None,
             out_dtype: torch.dtype = torch.bfloat16) -> torch.Tensor:
     """W4A16 linear ``x[..., K] -> [..., N]`` (bf16 in, fp32 accumulation; bf16 out, or the
     unrounded fp32 sums with ``out_dtype=torch.float32``)."""
-    if workspace is None and _plain(x) and (out_dtype is torch.bfloat16 or out_dtype is torch.float32):
-        y = _lib.host().linear(x, weight, out_dtype is torch.float32)
+    if (workspace is None and _plain(x) and (out_dtype is torch.bfloat16 or out_dtype is torch.float32)
+            and (host := _lib.host())):
+        y = host.linear(x, weight, out_dtype is torch.float32)
         if y is not None:
             return y
     weight.validate("weight")
@@ -193,16 +195,16 @@ def gdn_mixer(hidden: torch.Tensor, history: torch.Tensor, state: torch.Tensor, 
 def rms_norm(hidden: torch.Tensor, weight: torch.Tensor, eps: float) -> Optional[torch.Tensor]:
     """``layers.rms_normalise(hidden, weight, eps, 1.0)`` of a plain fp32 residual ``[T, H]`` in one launch; None for other
     forms (and where autograd follows it)."""
-    return _lib.host().rms_norm(hidden, weight, eps) if _plain(hidden) else None
+    return host.rms_norm(hidden, weight, eps) if _plain(hidden) and (host := _lib.host()) else None
 
 
 def gdn_mixer_plain(hidden, history, state, *, in_proj, out_proj, input_norm, post_norm, norm, a_log, dt_bias, conv,
                     key_heads, eps) -> Optional[GdnMixer]:
     """:func:`gdn_mixer` of arguments :func:`gdn_mixer_fits` accepts, both in one native call; None for others."""
-    if not _plain(hidden):
+    if not (_plain(hidden) and (host := _lib.host())):
         return None
-    r = _lib.host().gdn(hidden, history, state, in_proj, out_proj, input_norm, post_norm, norm, a_log, dt_bias, conv,
-                        key_heads, eps)
+    r = host.gdn(hidden, history, state, in_proj, out_proj, input_norm, post_norm, norm, a_log, dt_bias, conv, key_heads,
+                 eps)
     return None if r is None else GdnMixer(*r)
 
 
@@ -210,10 +212,10 @@ def attention_mixer_plain(hidden, keys, values, position, *, in_proj, out_proj, 
                           inv_freq, heads, kv_heads, head_dim, eps) -> Optional[tuple]:
     """:func:`attention_mixer` of arguments :func:`attention_mixer_fits` accepts, both in one native call; None for
     others."""
-    if not _plain(hidden):
+    if not (_plain(hidden) and (host := _lib.host())):
         return None
-    return _lib.host().attention(hidden, keys, values, position, in_proj, out_proj, input_norm, post_norm, q_norm, k_norm,
-                                 inv_freq, heads, kv_heads, head_dim, eps)
+    return host.attention(hidden, keys, values, position, in_proj, out_proj, input_norm, post_norm, q_norm, k_norm,
+                          inv_freq, heads, kv_heads, head_dim, eps)
 
 
 def _as(t, dtype: torch.dtype, shape: tuple, device: torch.device) -> bool:
@@ -268,8 +270,8 @@ def gdn_commit(state: torch.Tensor, keys: torch.Tensor, u: torch.Tensor, cum: to
     """``(recurrent state, conv history)`` after the first ``accepted`` tokens of one chunk of :func:`gdn_mixer`
     (``layers.state_after`` and the window's columns ``[first, first + 3)``) in one launch; ``None`` when the tensors
     are not laid out as that call leaves them, or autograd follows them."""
-    if _plain(state):
-        done = _lib.host().commit(state, keys, u, cum, accepted, window, first)
+    if _plain(state) and (host := _lib.host()):
+        done = host.commit(state, keys, u, cum, accepted, window, first)
         if done is not None:
             return done
     hv, device = state.shape[1], state.device
@@ -453,8 +455,8 @@ def moe_w4a16(hidden: torch.Tensor, gate_up: PackedW4, down: PackedW4, *, top_k:
     With ``return_routing=True`` also returns ``(Routing, logits)``; ``logits``
     are the fp32 router logits the routing was computed from.
     """
-    if router_logits is None and not return_routing and _plain(hidden):
-        out = _lib.host().moe(hidden, gate_up, down, top_k, router_weight, shared, workspace, None)
+    if router_logits is None and not return_routing and _plain(hidden) and (host := _lib.host()):
+        out = host.moe(hidden, gate_up, down, top_k, router_weight, shared, workspace, None)
         if out is not None:
             return out
     device, flat, sgu, sdn, sgate = _moe_common(hidden, gate_up, down, shared)
@@ -497,8 +499,8 @@ def moe_w4a16_add(residual: torch.Tensor, hidden: torch.Tensor, gate_up: PackedW
                   workspace: Optional[torch.Tensor] = None) -> torch.Tensor:
     """``residual + moe_w4a16(hidden, ...)`` in fp32 ``[T, H]`` without a launch for the add; ``residual`` is contiguous
     fp32 of hidden's shape."""
-    if _plain(hidden):
-        out = _lib.host().moe(hidden, gate_up, down, top_k, router_weight, shared, workspace, residual)
+    if _plain(hidden) and (host := _lib.host()):
+        out = host.moe(hidden, gate_up, down, top_k, router_weight, shared, workspace, residual)
         if out is not None:
             return out
     device, flat, sgu, sdn, sgate = _moe_common(hidden, gate_up, down, shared)
