@@ -14,9 +14,11 @@
 // spans few tokens.
 //
 // Bound by latency at verify sizes (T = 16 behind 4001 keys, 16 heads over 2 KV heads of 256: 8.4 MB of cache, 1.7 us at
-// the copy rate): prep 4.5, split 15.3 (19.0 with the row tiles of a split spread over the XCDs), combine 4.8 (9.8 with the
+// the copy rate): prep 4.1, split 15.8 (19.0 with the row tiles of a split spread over the XCDs), combine 5.3 (9.8 with the
 // splits read one after the other), in place of 60 library launches (250 us).  Against 64
 // bits the attention output is 4e-7 to 7e-7 off (fp32 library products 4e-7 to 1.8e-6).
+//
+// NaN and infinities as in a softmax over the visible keys: a NaN score makes its row NaN, a score of -inf has weight 0.
 #include <algorithm>
 
 #include "kernels.h"

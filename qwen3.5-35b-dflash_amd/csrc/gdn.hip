@@ -85,8 +85,8 @@ __global__ __launch_bounds__(512) void add_norm_kernel(const float* hidden, cons
 // ------------------------------------------------------------------ chunk preparation
 // Latency-bound at one chunk (32 workgroups): a wave per token, so conv, SiLU and the Q/K normalisation stay in
 // registers; then the two 16 x 16 products on one wave each beside the decay table, then the solve on four waves, while
-// the other waves write what does not depend on it.  T = 16, 32 heads: 9.6 us (17.0 us with four waves a
-// workgroup, each doing every phase, the window written last); T = 600: 32 us.
+// the other waves write what does not depend on it.  T = 16, 32 heads: 10 us (17 us with four waves a
+// workgroup, each doing every phase, the window written last); T = 600: 31 us.
 __global__ __launch_bounds__(1024) void gdn_chunk_kernel(GdnParams p) {
   __shared__ __align__(16) float qs[kChunk * kRow], ks[kChunk * kRow], vs[kChunk * kRow];
   __shared__ __align__(16) uint16_t raw[3][kChunk + kTaps - 1][kD + 2];  // window columns t0 - 3 .. t0 + 15
@@ -274,8 +274,8 @@ __global__ __launch_bounds__(1024) void gdn_chunk_kernel(GdnParams p) {
 // Four waves share a 128 x 16 state slice, wave w rows 32 w .. 32 w + 31: register (m, e) of lane l is row
 // 32 w + 16 m + 4 (l >> 4) + e, column l & 15, the result layout of the fp32 MFMA and, with the reduction taken in that
 // order of rows, also its B operand, so the state never leaves registers between chunks.  A 16-column slice is the
-// narrowest MFMA tile: 256 workgroups at 32 heads, one per CU.  T = 16: 4.5 us; T = 600 (38 chunks in series, 80 MB of
-// states written): 50 us, against about 4000 us for the same chunks as batched library products.
+// narrowest MFMA tile: 256 workgroups at 32 heads, one per CU.  T = 16: 5 us; T = 600 (38 chunks in series, 80 MB of
+// states written): 48 us, against about 4000 us for the same chunks as batched library products.
 __global__ __launch_bounds__(256) void gdn_state_kernel(GdnParams p) {
   __shared__ f32x4 part[2][2][4][64];  // [buffer][W S, Q~ S][wave][lane]
   const int h = blockIdx.x % p.Hv, slice = blockIdx.x / p.Hv;  // a head's slices share an XCD when Hv % 8 == 0

@@ -9,17 +9,18 @@
 //       weight is dequantised once per tile.  Activations reach LDS by direct-to-LDS loads, double buffered, one
 //       barrier per k-block; weights go straight into registers a k-block ahead.  168 registers and 33 KB of LDS:
 //       three workgroups share a CU, one computing while another waits at its barrier (against two: 2048 x 12288 x
-//       8192 441 -> 352 us, 2048 x 12352 x 2048 118 -> 113 us; 96-row tiles at two a CU 398 and 121 us).
+//       8192 441 -> 352 us, 2048 x 12352 x 2048 118 -> 113 us each alone; 96-row tiles at two a CU 398 and 121 us).
 //       The MFMAs accumulate into u, the running sum in units of the current group's scale: u is rescaled by
 //       s_prev / s at each k-block in the FMA that adds the offset term, which saves a second accumulator set.
 //       A wave that meets a scale which is no unit (zero, tiny, huge, not finite) takes its columns once more without.
 //       Bound by power: in the k-loop a workgroup takes 1509 cycles a k-block where the matrix core needs 1024, at a clock
-//       that falls from 2.4 to about 1.6 GHz.  2048 x 12352 x 2048: 113 us, 0.92 PFLOP/s (bf16 library product of that
-//       size 102 us; the 16-column streaming kernel that served these sizes before 267 us; 105 us among other calls).
+//       that falls from 2.4 to about 1.6 GHz.  2048 x 12352 x 2048 with the prep launch: 106 to 109 us among other calls,
+//       0.95 to 0.98 PFLOP/s (bf16 library product of that size 102 us; the 16-column streaming kernel that served these
+//       sizes before 267 us).  A zero scale in one column of every 64, so every wave twice: 269 us.
 //   w4_linear_split_kernel  for outputs of few tiles: a workgroup takes 32 rows x 64 columns, its four waves every fourth
 //       k-block each, operands straight into MFMA fragment registers, the four partial sums added in LDS in wave order.
-//       Bound by the latency of its loads: 333 x 2048 x 4096 in 24 us with the prep launch (4 us), 495 us on the
-//       per-wave kernel before.
+//       Bound by the latency of its loads: 333 x 2048 x 4096 in 23.0 us with the prep launch (kernel trace: 17.8 + 6.2),
+//       495 us on the per-wave kernel before.
 //
 // The line between them: tile when its tiles fill at least 5/8 of the CUs.  Measured, split / tile, us: 80 tiles 17.7 /
 // 22.9 (300 x 4096 x 2048) and 33.1 / 50.5 (600 x 2048 x 4096, portable); 160 tiles 25.2 / 25.2 (600 x 4096 x 2048); 196
@@ -382,7 +383,7 @@ __global__ __launch_bounds__(256, 3) void w4_linear_tile_kernel(LinearParams p) 
 // ------------------------------------------------------------------ k split over the waves
 // kStaged (portable banks): a wave's weights of a k-block reach LDS by four direct-to-LDS loads of 16 whole 64-byte row
 // pieces each, and lanes read their fragments from there; straight into registers each load would take 32 bytes of 32
-// rows (333 x 2048 x 4096 28.7 -> 24.1 us, 600 x 2048 x 4096 39.3 -> 33.1).  Tiled banks lie in fragment order already.
+// rows (333 x 2048 x 4096 27.6 -> 23.0 us, 600 x 2048 x 4096 39.3 -> 33.1).  Tiled banks lie in fragment order already.
 template <typename ScaleT, bool kStaged>
 __global__ __launch_bounds__(256, 2) void w4_linear_split_kernel(LinearParams p) {
   __shared__ f32x4 part[4][8][64];  // a wave's eight kilobytes are also its two weight stages, [64 rows][4 pieces] each
