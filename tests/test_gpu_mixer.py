@@ -392,14 +392,13 @@ def test_attention_kernels_keep_fp32(pkg, device, tokens, context, heads, kv_hea
 
 
 @pytest.mark.parametrize("kind", ["linear_attention", "full_attention"])
-@pytest.mark.parametrize("tokens", [1, 9, 32, 40])
-@pytest.mark.parametrize("group,scale_dtype,layout", [(256, torch.float32, "portable"), (256, torch.float32, "tiled"),
-                                                      (128, torch.bfloat16, "portable")])
+@pytest.mark.parametrize("group,scale_dtype,layout,tokens", [
+    (group, dtype, layout, tokens)
+    for group, dtype, layout in ((256, torch.float32, "portable"), (256, torch.float32, "tiled"), (128, torch.bfloat16, "portable"))
+    for tokens in (1, 9, 32, 40) if layout == "portable" or tokens <= 32])    # tiled groups of 256 end at 32 rows
 def test_mixers_over_other_banks(pkg, device, kind, tokens, group, scale_dtype, layout):
     """Groups of 256, fp32 scales and the portable layout through both mixers, against the PyTorch form on the same banks:
     both run the same projections, so what differs is fp32 sums between them and bf16 roundings that follow."""
-    if layout == "tiled" and tokens > 32:
-        pytest.skip("tiled groups of 256 above 32 rows have no kernel")
     c = pkg.target.small_config((kind,))
     model = pkg.target.TargetModel(pkg.target.random_weights(c, seed=9, device=device, layout="portable"), capacity=96)
     lw, gen = model.w.layers[0], torch.Generator().manual_seed(group + tokens)
@@ -418,3 +417,43 @@ def test_mixers_over_other_banks(pkg, device, kind, tokens, group, scale_dtype, 
     else:
         general = model._attention(normed, lw, other.keys[0], other.values[0], 21)
     assert metrics.compare((trace["mid"] - x).cpu(), general.float().cpu())["max_rel"] <= TOL
+
+
+def _forms(tensor):
+    """Other forms of a tensor: another type, shape, order in memory and alignment."""
+    flat = torch.zeros((tensor.numel() + 1,), dtype=tensor.dtype, device=tensor.device)[1:].view(tensor.shape)
+    strided = torch.zeros((*tensor.shape, 2), dtype=tensor.dtype, device=tensor.device)[..., 0]
+    return [tensor.double(), tensor[..., :-1].contiguous(), strided, flat, tensor.cpu(), tensor.detach().requires_grad_()]
+
+
+@pytest.mark.parametrize("kind", ["linear_attention", "full_attention"])
+def test_the_native_mixers_take_what_the_python_form_takes(pkg, device, kind):
+    """Both say which calls the kernels get: the plain one, and neither any other form of an argument."""
+    c = pkg.target.small_config((kind,))
+    model = pkg.target.TargetModel(pkg.target.random_weights(c, seed=9, device=device), capacity=32)
+    lw, state, x = model.w.layers[0], model.synthetic_context(9, seed=4), torch.randn((4, c.hidden), device=device)
+    if kind == "linear_attention":
+        args = dict(hidden=x, history=state.conv[0], state=state.recurrent[0], **model._gdn_args(lw))
+        plain, fits = pkg.ops.gdn_mixer_plain, pkg.ops.gdn_mixer_fits
+        others = dict(key_heads=[3, 32])
+    else:
+        args = dict(hidden=x, keys=state.keys[0], values=state.values[0], position=9, in_proj=lw.mixer_in,
+                    out_proj=lw.mixer_out, input_norm=lw.input_norm, post_norm=lw.post_norm, q_norm=lw.q_norm,
+                    k_norm=lw.k_norm, inv_freq=model.inv_freq, heads=4, kv_heads=2, head_dim=128, eps=1e-6)
+        plain, fits = pkg.ops.attention_mixer_plain, pkg.ops.attention_mixer_fits
+        others = dict(position=[29], heads=[8], kv_heads=[1, 4], head_dim=[256, 64])
+    assert plain(**args) is not None and fits(**args)
+    others["in_proj"] = [args["out_proj"], args["in_proj"]._replace(packed=args["in_proj"].packed[:-32])]
+    others["out_proj"] = [args["in_proj"]]
+    for name, value in args.items():
+        if isinstance(value, torch.Tensor):
+            others[name] = _forms(value)
+    for name, values in others.items():
+        for value in values:
+            call = {**args, name: value}
+            native = plain(**call) is not None
+            try:
+                python = fits(**call)
+            except ValueError:                          # a bank that is no bank
+                python = False
+            assert not native and not python, (name, getattr(value, "dtype", value), getattr(value, "shape", None))
