@@ -1313,8 +1313,13 @@ int dflash_moe_w4a16_residual(const void* hidden, int64_t tokens, int64_t hidden
                               const void* shared_gate_weight, const float* residual, float* sum, float* logits_out,
                               int32_t* topk_ids, float* topk_weights, int32_t* perm, int32_t* inv_perm,
                               int32_t* expert_offsets, void* workspace, size_t workspace_bytes, void* stream) {
-  if (!residual || !sum || !aligned16(residual) || !aligned16(sum))
-    return fail(DFLASH_ERR_INVALID_ARGUMENT, "moe_residual: residual and sum NULL or not 16-byte aligned");
+  if (!residual || !sum || !aligned16(residual) || !aligned16(sum)) {
+    try {
+      return fail(DFLASH_ERR_INVALID_ARGUMENT, "moe_residual: residual and sum NULL or not 16-byte aligned");
+    } catch (...) {  // no memory for the message
+      return DFLASH_ERR_INVALID_ARGUMENT;
+    }
+  }
   return moe_w4a16_body(hidden, tokens, hidden_size, nullptr, router_weight, top_k, gate_up, down, shared_gate_up,
                         shared_down, shared_gate_weight, nullptr, logits_out, topk_ids, topk_weights, perm, inv_perm,
                         expert_offsets, workspace, workspace_bytes, false, stream, residual, sum);

@@ -394,3 +394,14 @@ def test_mixers_refuse_a_projection_without_a_kernel(pkg):
             input_norm=v, post_norm=v, norm=v, a_log=v, dt_bias=v, conv=v, hidden_size=512, key_heads=hk, value_heads=hv, eps=1e-6)
         st, msg = _status(pkg, "dflash_gdn_mixer", ctypes.byref(desc), v, tokens, v, v, v, v, v, v, v, v, v, v, v, v, 16, None)
         assert (st, why in msg) == (2, True) if why else (st, "workspace" in msg) == (3, True)
+
+
+@host_only
+@pytest.mark.parametrize("residual,out", [(None, 16), (16, None), (24, 16), (16, 24)])
+def test_moe_residual_validation(pkg, residual, out):
+    """NULL or misaligned residual and sum are refused on the host."""
+    p = ctypes.c_void_p(16)
+    gu, dn = _desc(pkg, experts=256, rows=1024, cols=2048), _desc(pkg, experts=256, rows=2048, cols=512)
+    st, msg = _status(pkg, "dflash_moe_w4a16_residual", p, 16, 2048, p, 8, ctypes.byref(gu), ctypes.byref(dn), None, None, None,
+                      ctypes.c_void_p(residual), ctypes.c_void_p(out), p, p, p, p, p, p, p, 1 << 30, None)
+    assert st == 1 and "residual" in msg
